@@ -8,13 +8,10 @@
 // each XCD owns a contiguous run of output tiles (consecutive tiles share a
 // weight column-block, so its dequantised slabs are served from that XCD's L2).
 #include "gemm.hpp"
+#include "gemm_common.hpp"
 
 namespace pkx {
 
-
-// Rows of each 64-wide K slab block of a slab-major (q8_0 / q4_K) weight (views
-// into a larger allocation keep the allocation's row count).
-__device__ __forceinline__ int slab_rows(const GemmParams& p) { return p.ldw > 0 ? p.ldw : p.N; }
 
 // The arguments every GEMM prologue reads, pulled into SGPRs in one batch of
 // scalar loads at kernel entry.  Left to itself the compiler loads the
@@ -28,70 +25,6 @@ __device__ __forceinline__ void prefetch_gemm_args(const GemmParams& p) {
 
 // Wave index as a wave-uniform (scalar) value.
 __device__ __forceinline__ int wave_id_uniform() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
-
-// 2-D XCD blocking: the nbm x nbn tile grid is cut into gm row bands x gn
-// column bands (gm * gn = 8), one rectangle per XCD, so an XCD's L2 sees only
-// its band of A rows and its band of weight columns (gn*|A| + gm*|W| bytes
-// over the chip instead of 8*|A| or 8*|W|).  xcd_tile gives each XCD a
-// contiguous range of positions; positions enumerate the rectangles in order,
-// each rectangle M-fastest, so the map is a bijection for any grid size.
-// gm and gn are powers of two, so the band edges i * nbm / gm are shifts; the
-// one division left is the split of k inside its rectangle.  (With a division
-// for every band edge this ran ~3k cycles at the start of every launch, all
-// of it before the first load: 32-bit division by a runtime value is a
-// ~40-instruction scalar / vector round trip on this hardware.)
-__device__ __forceinline__ void xcd_rect(int k, int nbm, int nbn, int gm, int& bm, int& bn) {
-    const int lgm = __builtin_ctz(gm), lgn = 3 - lgm;
-    for (int i = 0; i < gm; ++i) {
-        const int r0 = (i * nbm) >> lgm, r1 = ((i + 1) * nbm) >> lgm;
-        for (int j = 0; j < (1 << lgn); ++j) {
-            const int c0 = (j * nbn) >> lgn, c1 = ((j + 1) * nbn) >> lgn;
-            const int h = r1 - r0, sz = h * (c1 - c0);
-            if (k < sz) {   // sz > 0, so h > 0
-                const int q = (int)((unsigned)k / (unsigned)h);
-                bm = r0 + (k - q * h);
-                bn = c0 + q;
-                return;
-            }
-            k -= sz;
-        }
-    }
-    bm = bn = 0;   // unreachable: the rectangles cover the grid
-}
-__device__ __forceinline__ void xcd_tile_2d(int bid, int nbm, int nbn, int gm, int& bm, int& bn) {
-    xcd_rect(xcd_tile(bid, nbm * nbn), nbm, nbn, gm, bm, bn);
-}
-
-// ---------------------------------------------------------------------------
-// Epilogue for one accumulator element (everything except GLU).
-// ---------------------------------------------------------------------------
-template <int EPI, typename ActT>
-__device__ __forceinline__ void epi_one(const GemmParams& p, int m, int n, float acc) {
-    float v = acc + (p.bias ? p.bias[n] : 0.0f);
-    if constexpr (EPI == EPI_STORE) {
-        ((ActT*)p.Y)[(int64_t)m * p.ldy + n] = to_act<ActT>(v * p.alpha);
-    } else if constexpr (EPI == EPI_STORE_F32) {
-        ((float*)p.Y)[(int64_t)m * p.ldy + n] = v * p.alpha;
-    } else if constexpr (EPI == EPI_SILU) {
-        ((ActT*)p.Y)[(int64_t)m * p.ldy + n] = to_act<ActT>(silu_dev(v));
-    } else if constexpr (EPI == EPI_RESID) {
-        float* r = (float*)p.Y + (int64_t)m * p.ldy + n;
-        *r = *r + v * p.alpha;
-    } else if constexpr (EPI == EPI_RELU) {
-        ((ActT*)p.Y)[(int64_t)m * p.ldy + n] = to_act<ActT>(v > 0.f ? v : 0.f);
-    } else if constexpr (EPI == EPI_RELU_TR) {
-        // rows are pixels (b, t, f), f fastest; store [b][t][c][f] (channel-major flatten)
-        const int F = p.trF;
-        const int bt = m / F, f = m - bt * F;
-        const int t = bt % p.T, b = bt / p.T;
-        float o = v > 0.f ? v : 0.f;
-        if (p.valid && t >= p.valid[b]) o = 0.f;
-        ((ActT*)p.Y)[((int64_t)bt * p.N + n) * F + f] = to_act<ActT>(o);
-    } else if constexpr (EPI == EPI_RELU2_F32) {
-        float o = v + (p.bias2 ? p.bias2[n] : 0.0f);
-        ((float*)p.Y)[(int64_t)m * p.ldy + n] = o > 0.f ? o : 0.f;
-    }
-}
 
 template <int EPI, typename ActT, int TM, int TN>
 __device__ __forceinline__ void epilogue(const GemmParams& p, float4v (&acc)[TM][TN], int mw,
@@ -2874,11 +2807,14 @@ void launch_gemm(Precision prec, int wtype, int epi, const GemmParams& p, hipStr
         default: throw std::invalid_argument("gemm(f16): weight type must be f16/q8_0/q4_K");
         }
     } else {
-        // 64x128 tiles while they fill the chip; a single utterance (M = T' ~ 125)
-        // gives only 8-32 of them, so smaller tiles buy workgroups there
-        const int64_t t24 = (int64_t)cdiv(p.M, 64) * cdiv(p.N, 128);
+        if (wtype == GT_F32 && launch_gemm_f32_ks(epi, p, s)) return;
+        // 64x128 tiles when their last round of the chip is at least 90% full (M = 2000,
+        // N = 2048, K = 512: 512 tiles 51.6 us against 56.2 with 32x64; N = 1025, K = 1024: 288
+        // tiles, a second round for 32 of them, 86.6 against 61.9), else 32x64 while those
+        // fill the chip, else 32x32
+        const int64_t t24 = (int64_t)cdiv(p.M, 64) * cdiv(p.N, 128), cus = device_cu_count();
         const int64_t t12 = (int64_t)cdiv(p.M, 32) * cdiv(p.N, 64);
-        const int shape = t24 >= 256 ? 0 : t12 >= 256 ? 1 : 2;
+        const int shape = t24 >= 256 && 10 * t24 >= 9 * cus * cdiv(t24, cus) ? 0 : t12 >= 256 ? 1 : 2;
         switch (wtype) {
         case GT_F32: f32_shape<GT_F32>(shape, epi, p, s); break;
         case GT_F16: f32_shape<GT_F16>(shape, epi, p, s); break;

@@ -183,3 +183,29 @@ def test_residual_two_k_groups(gpu, stream, gtype, K):
     _residual_calls(gpu, stream, gtype, K, ((2000, 1024), (2040, 1024), (1990, 1024), (2000, 960)),
                     _rng(K + gtype), "two-k-groups")
 
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 33, 8), (17, 31, 1000), (125, 512, 2048), (16, 32, 1024), (249, 2048, 520),
+                                   (33, 1025, 40), (1000, 1030, 1032), (700, 512, 512), (513, 640, 1024)])
+def test_linear_f32_k_split(gpu, stream, M, N, K):
+    """f32 weights on the K-split tiles (16 x 32 with four and eight K groups,
+    32 x 32 with four): partial tiles on both edges, K that is no whole number
+    of 32-column steps, fewer steps than K groups.  Every element within the
+    worst-case f32 summation bound of the float64 product, for the store and
+    for the residual update."""
+    rng = _rng(M + 3 * N + K)
+    w = rng.normal(0, 0.05, (N, K)).astype(np.float32)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    b = rng.normal(0, 0.1, N).astype(np.float32)
+    y0 = rng.normal(0, 1, (M, N)).astype(np.float32)
+    print(f"[linear-f32-ks] M={M} N={N} K={K}", flush=True)
+    acc = x.astype(np.float64) @ w.T.astype(np.float64) + b
+    bound = K * 2.0 ** -24 * (np.abs(x).astype(np.float64) @ np.abs(w).T) + 2.0 ** -22 * (np.abs(acc) + 1.0)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    db = gpu.DeviceArray.from_numpy(b, stream)
+    dy = gpu.DeviceArray((M, N), np.float32)
+    gpu.linear(0, pm.GGML_F32, N, K, w, dx, M, dy, db, stream)
+    assert (np.abs(dy.numpy(stream) - acc) <= bound).all()
+    dr = gpu.DeviceArray.from_numpy(y0, stream)
+    gpu.linear_residual(0, pm.GGML_F32, N, K, w, dx, M, dr, 0.5, db, stream)
+    assert (np.abs(dr.numpy(stream) - (y0 + 0.5 * acc)) <= bound + 2.0 ** -22 * np.abs(y0)).all()
