@@ -9,10 +9,18 @@
 // the twiddle table is the reference's own recurrence, built on the host), so
 // per-frame results match the reference's up to the libm ulp of sqrt/pow/log.
 //
-// mel_spec_kernel: one workgroup per (16 frames, clip); each wave runs the
-// FFT of one frame at a time in LDS (complex f64), keeps the frame's power
-// spectrum in LDS, then the workgroup computes the 16 x n_mels filterbank sums
-// (one f64 chain per output, summed in bin order) and writes log-mel.
+// mel_spec512_kernel (n_fft 512, mag_power 2, a filterbank that fits its LDS): persistent workgroups over groups of four
+// frames of a clip, a frame a wave.  The frame's 512 real samples are a 256-point complex
+// FFT (x[2n] + i x[2n+1]) of four radix-4 stages, four values per lane in
+// registers and one LDS exchange between stages, then split into the 257 bins.
+// It rounds differently from the reference's radix-2 butterflies, by f64 ulps
+// (fewer operations; error against f128 no larger), far below the f32 rounding
+// of the bins.
+// mel_spec_kernel (everything else): each wave runs the reference's butterflies on
+// one frame at a time in LDS (complex f64).
+// Both keep the frames' power spectra in LDS; the workgroup then computes the
+// filterbank sums of its frames (one f64 chain per output, summed in bin order)
+// and writes log-mel.
 // mel_norm_kernel: one workgroup per (mel bin, clip): per-feature mean and
 // unbiased std over the clip's first S/hop frames, normalisation, zeroing of
 // the rest of the row up to T_max.
@@ -30,17 +38,228 @@ namespace pkx {
 struct MelParams {
     const float* pcm;
     int64_t S_stride;
-    const int* meta;           // [B][2]: samples, frames
+    const int* meta;           // samples of each clip, or null: in inl
+    int inl[MEL_INLINE_CLIPS];
     const float* window;       // [n_fft]
     const float* fb;           // [n_mels][n_bins]
     const double* tw;          // [n_fft - 1][2]: stage of half-length h uses rows h-1 .. 2h-2
+    const double* tw512;       // n_fft 512: [512][2] = exp(-2 pi i k / 512)
     const int4* span;          // [n_mels]: the filter's nonzero bins [x, y), packed offset z
     const float* fb_packed;    // the filters' values over their spans, back to back
     int fb_nnz;
     float* out;                // [B][n_mels][T_max]
     int T_max, n_fft, log2n, hop, n_mels, n_bins, per_feature;
     float preemph, mag_power, log_guard;
+    __device__ __forceinline__ int samples(int b) const { return meta ? meta[b] : inl[b]; }
+    // frames of an S-sample clip (MelFront::frames)
+    __device__ __forceinline__ int frames(int S) const { return S <= 0 || S + 2 * (n_fft / 2) < n_fft ? 0 : 1 + (S + 2 * (n_fft / 2) - n_fft) / hop; }
 };
+
+// Filterbank + log (src/mel.cpp:82-89) of a workgroup's FB frames, one f64
+// chain per output summed in bin order over the filter's nonzero span only:
+// every other bin would add fb * power = +-0, which leaves the sum unchanged.
+// Four bins' operands are read at a time (LDS latency is what bounds the
+// chain).  Output (m, f) with f fastest.
+// LDS: the filter values are in fbs.
+template <int FB, bool LDS>
+__device__ __forceinline__ void mel_bank(const MelParams& p, const double (*pw)[MEL_MAX_NFFT / 2 + 1], const float* fbs,
+                                         const int4* spans, int b, int t0, int T) {
+    const int tid = threadIdx.x, f = tid & (FB - 1), t = t0 + f;
+    for (int m = tid / FB; m < p.n_mels; m += 256 / FB) {
+        const int4 sp = spans[m];   // {first bin, end bin, packed offset, -}
+        double acc = 0.0;
+        auto run = [&](const float* w) {
+            for (int k = sp.x; k < sp.y; k += 4) {
+                float wv[4];
+                double pv[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int kk = min(k + e, sp.y - 1);
+                    wv[e] = w[kk - sp.x];
+                    pv[e] = pw[f][kk];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (k + e < sp.y) acc += (double)wv[e] * pv[e];
+            }
+        };
+        if constexpr (LDS) run(fbs + sp.z);
+        else run(p.fb_packed + sp.z);
+        if (t < T) p.out[((int64_t)b * p.n_mels + m) * p.T_max + t] = (float)log(acc + (double)p.log_guard);
+    }
+}
+
+// The power of one bin from its f32-rounded value (src/mel.cpp:73-79, fft.cpp:70-71).
+// pow(sqrt(x), 2) is x up to its own rounding: mag_power 2 takes x.
+__device__ __forceinline__ double sq_abs(double re64, double im64) {
+    const float re = (float)re64, im = (float)im64;
+    return (double)re * re + (double)im * im;
+}
+__device__ __forceinline__ double mel_power(const MelParams& p, double re64, double im64) {
+    const double sq = sq_abs(re64, im64);
+    if (p.mag_power == 2.0f) return sq;
+    const double mag = sqrt(sq);
+    return p.mag_power == 1.0f ? mag : pow(mag, (double)p.mag_power);
+}
+
+struct Cplx {
+    double x, y;
+};
+__device__ __forceinline__ Cplx operator+(Cplx a, Cplx b) { return {a.x + b.x, a.y + b.y}; }
+__device__ __forceinline__ Cplx operator-(Cplx a, Cplx b) { return {a.x - b.x, a.y - b.y}; }
+__device__ __forceinline__ Cplx cmul(Cplx a, Cplx b) {
+    return {fma(a.x, b.x, -(a.y * b.y)), fma(a.x, b.y, a.y * b.x)};
+}
+
+// A workgroup takes groups of four frames, one a wave, gridDim.x apart in the
+// order (clip, frame): its twiddles, window, filter spans and weights are loaded
+// once, and the next group's samples are on their way while the current one
+// computes.  What bounds it is VALU issue (about 700 instructions a wave and
+// frame, most of them f64 at a quarter rate: half of the time) and the LDS
+// exchanges' latency, four waves a SIMD.  16 x 10 s, 128 filters on MI355X:
+// 39 us; the radix-2 butterflies through LDS with pow() 152; this FFT with one
+// group of four frames a workgroup 50, of eight 60 (two waves a SIMD).
+__global__ __launch_bounds__(256, 4) void mel_spec512_kernel(MelParams p, int groups, int n_groups) {
+    constexpr int FB = 4;
+    constexpr int LEN = 256 + 256 / 32;        // one pad per 32 values: the stage writes spread over the banks
+    __shared__ double ex[4][2][LEN];           // per wave: re, im
+    __shared__ double pws[2][FB][MEL_MAX_NFFT / 2 + 1];
+    __shared__ int4 sps[MEL_SPAN_LDS];
+    __shared__ float2v wins[256];
+    __shared__ float fbs[MEL_FB_LDS];
+    const int tid = threadIdx.x, j = tid & 63, w = tid >> 6;
+    const double pre = (double)p.preemph;
+
+    // samples q - 1, q, q + 1 of n = j + 64 r, q = 2n past the frame's start (groups: frame groups of a clip)
+    // (inside: every sample of this wave's frame and the one before it exist)
+    struct Group {
+        int b, t0, S, T;
+        bool inside;
+    };
+    float v[4][3];
+    auto fetch = [&](int g) {
+        Group u;
+        u.b = g / groups;
+        u.t0 = (g - u.b * groups) * FB;
+        u.S = p.samples(u.b);
+        u.T = p.frames(u.S);
+        const float* x = p.pcm + (int64_t)u.b * p.S_stride;
+        const int q0 = __builtin_amdgcn_readfirstlane((u.t0 + w) * p.hop - 256);
+        u.inside = q0 > 0 && q0 + 512 <= u.S;
+        if (u.inside) {
+            x += q0 + 2 * j;
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int e = 0; e < 3; ++e) v[r][e] = x[128 * r + e - 1];
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int q = q0 + 2 * (j + 64 * r);
+#pragma unroll
+                for (int e = 0; e < 3; ++e)
+                    v[r][e] = u.t0 + w < u.T && q + e - 1 >= 0 && q + e - 1 < u.S ? x[q + e - 1] : 0.0f;
+            }
+        }
+        return u;
+    };
+    int g = blockIdx.x;
+    Group cur = fetch(g);
+    wins[tid] = *(const float2v*)(p.window + 2 * tid);
+    // twiddles: stage s (butterfly span N = 4^s, s = 1..3) exp(-2 pi i r (j % N) / 4N), and the split's
+    // exp(-2 pi i k / 512), k = j, j + 64
+    auto tw = [&](int k) { return Cplx{p.tw512[2 * k], p.tw512[2 * k + 1]}; };
+    Cplx ts[3][3], tk[2];
+#pragma unroll
+    for (int s = 0; s < 3; ++s)
+#pragma unroll
+        for (int r = 1; r < 4; ++r) ts[s][r - 1] = tw((r * (j & ((4 << (2 * s)) - 1)) * (32 >> (2 * s))) & 511);
+    tk[0] = tw(j);
+    tk[1] = tw(j + 64);
+    for (int i = tid; i < p.n_mels; i += 256) sps[i] = p.span[i];
+    for (int i = tid; i < p.fb_nnz; i += 256) fbs[i] = p.fb_packed[i];
+    __syncthreads();
+
+    double *er = ex[w][0], *ei = ex[w][1];
+    auto at = [](int i) { return i + (i >> 5); };
+    // the wave's LDS operations complete in order: these only keep the compiler's order
+    auto fence = [] { __builtin_amdgcn_wave_barrier(); asm volatile("" ::: "memory"); };
+    for (int buf = 0;; buf ^= 1) {
+        // windowed samples 2n, 2n + 1 (src/mel.cpp:67-69)
+        Cplx z[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int q = (cur.t0 + w) * p.hop + 2 * (j + 64 * r) - 256;
+            const float2v wn = wins[j + 64 * r];
+            float f[2];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                double d = (double)v[r][e + 1];
+                if (p.preemph > 0.0f && (cur.inside || (q + e > 0 && q + e < cur.S))) d = (double)v[r][e + 1] - pre * (double)v[r][e];
+                f[e] = (float)(d * (double)wn[e]);
+            }
+            z[r] = {(double)f[0], (double)f[1]};
+        }
+        const Group now = cur;
+        g += gridDim.x;
+        if (g < n_groups) cur = fetch(g);
+        if (now.t0 < now.T) {   // uniform over the workgroup
+            // Stockham stages: lane j takes values j + 64 r, leaves (j / N) 4N + j % N + r N
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const int N = 1 << (2 * s);
+                if (s > 0) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) z[r] = {er[at(j + 64 * r)], ei[at(j + 64 * r)]};
+                    fence();
+#pragma unroll
+                    for (int r = 1; r < 4; ++r) z[r] = cmul(z[r], ts[s - 1][r - 1]);
+                }
+                const Cplx a = z[0] + z[2], c = z[0] - z[2], d = z[1] + z[3], e = z[1] - z[3];
+                z[0] = a + d;
+                z[2] = a - d;
+                z[1] = {c.x + e.y, c.y - e.x};   // c - i e
+                z[3] = {c.x - e.y, c.y + e.x};
+                const int base = (j / N) * 4 * N + (j & (N - 1));
+                if (s < 3) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) {
+                        er[at(base + r * N)] = z[r].x;
+                        ei[at(base + r * N)] = z[r].y;
+                    }
+                    fence();
+                }
+            }
+            // bins k and 256 - k from Z[k] and Z[256 - k]: this lane has k = j, j + 64 (r = 0, 1)
+            // and hands over 128 + j, 192 + j
+#pragma unroll
+            for (int r = 2; r < 4; ++r) {
+                er[at(64 * r + j)] = z[r].x;
+                ei[at(64 * r + j)] = z[r].y;
+            }
+            fence();
+            double* P = pws[buf][w];
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                const int k = j + 64 * r, kc = (256 - k) & 255;
+                Cplx c = {er[at(kc)], ei[at(kc)]};
+                if (k == 0) c = z[0];
+                const Cplx e = {0.5 * (z[r].x + c.x), 0.5 * (z[r].y - c.y)};      // even samples' bin
+                const Cplx o = {0.5 * (z[r].y + c.y), 0.5 * (c.x - z[r].x)};      // odd samples' bin
+                const Cplx x = cmul(o, tk[r]);
+                P[k] = sq_abs(e.x + x.x, e.y + x.y);
+                P[256 - k] = sq_abs(e.x - x.x, x.y - e.y);
+            }
+            if (j == 0) P[128] = sq_abs(z[2].x, -z[2].y);
+            fence();
+        }
+        // one barrier a group: the spectra alternate between two buffers, and every wave is past
+        // the filterbank of the group before when it writes this one's successor
+        __syncthreads();
+        if (now.t0 < now.T) mel_bank<FB, true>(p, pws[buf], fbs, sps, now.b, now.t0, now.T);
+        if (g >= n_groups) break;
+    }
+}
 
 __global__ __launch_bounds__(256) void mel_spec_kernel(MelParams p) {
     constexpr int FB = MEL_FRAMES_PER_BLOCK, RPL = MEL_MAX_NFFT / 64;
@@ -49,7 +268,7 @@ __global__ __launch_bounds__(256) void mel_spec_kernel(MelParams p) {
     __shared__ double2 tws[MEL_MAX_NFFT];
     __shared__ float fbs[MEL_FB_LDS];
     const int b = blockIdx.y, t0 = blockIdx.x * FB;
-    const int S = p.meta[2 * b], T = p.meta[2 * b + 1];
+    const int S = p.samples(b), T = p.frames(S);
     if (t0 >= T) return;                               // uniform over the workgroup
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int N = p.n_fft, pad = N / 2;
@@ -76,8 +295,7 @@ __global__ __launch_bounds__(256) void mel_spec_kernel(MelParams p) {
         }
     }
     for (int i = tid; i < N - 1; i += 256) tws[i] = make_double2(p.tw[2 * i], p.tw[2 * i + 1]);
-    const bool fb_lds = p.fb_nnz <= MEL_FB_LDS;
-    if (fb_lds)
+    if (p.fb_nnz <= MEL_FB_LDS)
         for (int i = tid; i < p.fb_nnz; i += 256) fbs[i] = p.fb_packed[i];
 
     for (int r = 0; r < FB / 4; ++r) {
@@ -103,29 +321,11 @@ __global__ __launch_bounds__(256) void mel_spec_kernel(MelParams p) {
             }
             __syncthreads();
         }
-        // power spectrum (src/mel.cpp:73-79): bins rounded to f32 first (fft.cpp:70-71)
-        for (int k = lane; k < p.n_bins; k += 64) {
-            const float re = (float)B2[k].x, im = (float)B2[k].y;
-            const double mag = sqrt((double)re * re + (double)im * im);
-            pw[f][k] = p.mag_power == 1.0f ? mag : pow(mag, (double)p.mag_power);
-        }
+        for (int k = lane; k < p.n_bins; k += 64) pw[f][k] = mel_power(p, B2[k].x, B2[k].y);
         __syncthreads();
     }
-    // filterbank + log (src/mel.cpp:82-89), one f64 chain per output summed
-    // in bin order over the filter's nonzero span only: every other bin would
-    // add fb * power = +-0, which leaves the sum unchanged, so the result is
-    // the reference's dense sum bit for bit.  Output (m, f) with f fastest.
-    const int f = tid & (FB - 1), t = t0 + f;
-    for (int m = tid / FB; m < p.n_mels; m += 256 / FB) {
-        const int4 sp = p.span[m];                     // {first bin, end bin, packed offset, -}
-        double acc = 0.0;
-        if (fb_lds) {
-            for (int k = sp.x; k < sp.y; ++k) acc += (double)fbs[sp.z + k - sp.x] * pw[f][k];
-        } else {
-            for (int k = sp.x; k < sp.y; ++k) acc += (double)p.fb_packed[sp.z + k - sp.x] * pw[f][k];
-        }
-        if (t < T) p.out[((int64_t)b * p.n_mels + m) * p.T_max + t] = (float)log(acc + (double)p.log_guard);
-    }
+    if (p.fb_nnz <= MEL_FB_LDS) mel_bank<FB, true>(p, pw, fbs, p.span, b, t0, T);
+    else mel_bank<FB, false>(p, pw, fbs, p.span, b, t0, T);
 }
 
 __device__ __forceinline__ double block_sum_f64(double v, double* red) {
@@ -137,27 +337,46 @@ __device__ __forceinline__ double block_sum_f64(double v, double* red) {
     return (red[0] + red[1]) + (red[2] + red[3]);
 }
 
+// Rows of up to 256 NV frames stay in registers between the passes (NV = 0:
+// longer ones are read again): what bounds the kernel is the latency of its
+// dependent passes over a row.
+template <int NV>
 __global__ __launch_bounds__(256) void mel_norm_kernel(MelParams p) {
     __shared__ double red[4];
     const int m = blockIdx.x, b = blockIdx.y;
-    const int S = p.meta[2 * b], T = p.meta[2 * b + 1];
+    const int S = p.samples(b), T = p.frames(S);
     float* row = p.out + ((int64_t)b * p.n_mels + m) * p.T_max;
     int keep = T;
     if (p.per_feature && T > 0) {
         // src/mel.cpp:157-182: mean and unbiased std over the first S/hop frames
         const int valid = min(S / p.hop, T);
+        float x[NV > 0 ? NV : 1];
+        if constexpr (NV > 0) {
+#pragma unroll
+            for (int i = 0; i < NV; ++i) x[i] = threadIdx.x + 256 * i < (unsigned)valid ? row[threadIdx.x + 256 * i] : 0.0f;
+        }
+        // f(frame, value) over this thread's frames, in order
+        auto each = [&](auto&& f) {
+            if constexpr (NV > 0) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+                    if (threadIdx.x + 256 * i < (unsigned)valid) f(threadIdx.x + 256 * i, x[i]);
+            } else {
+                for (int t = threadIdx.x; t < valid; t += 256) f(t, row[t]);
+            }
+        };
         double s = 0.0;
-        for (int t = threadIdx.x; t < valid; t += 256) s += (double)row[t];
+        each([&](int, float v) { s += (double)v; });
         const double mean = valid > 0 ? block_sum_f64(s, red) / (double)valid : 0.0;
         double q = 0.0;
-        for (int t = threadIdx.x; t < valid; t += 256) {
-            const double d = (double)row[t] - mean;
+        each([&](int, float v) {
+            const double d = (double)v - mean;
             q += d * d;
-        }
+        });
         const double ss = block_sum_f64(q, red);
         const double var = valid > 1 ? ss / (double)(valid - 1) : 0.0;
         const double sd = sqrt(var) + 1e-5;
-        for (int t = threadIdx.x; t < valid; t += 256) row[t] = (float)(((double)row[t] - mean) / sd);
+        each([&](int t, float v) { row[t] = (float)(((double)v - mean) / sd); });
         keep = valid;
     }
     for (int t = keep + threadIdx.x; t < p.T_max; t += 256) row[t] = 0.0f;
@@ -195,6 +414,16 @@ MelFront::MelFront(const MelConfig& c, const float* window, int win_len, const f
             ci = ni;
         }
     }
+    if (c.n_fft == 512) {
+        std::vector<double> t5(2 * 512);
+        for (int k = 0; k < 512; ++k) {
+            const double a = -2.0 * M_PI * k / 512;
+            t5[2 * (size_t)k] = std::cos(a);
+            t5[2 * (size_t)k + 1] = std::sin(a);
+        }
+        PKX_HIP(hipMalloc(&d_tw512_, sizeof(double) * t5.size()));
+        PKX_HIP(hipMemcpy(d_tw512_, t5.data(), sizeof(double) * t5.size(), hipMemcpyHostToDevice));
+    }
     // each filter's nonzero span and its values packed back to back (the
     // kernel skips the exact zeros outside the span)
     std::vector<int4> span((size_t)c.n_mels);
@@ -225,7 +454,7 @@ MelFront::MelFront(const MelConfig& c, const float* window, int win_len, const f
 }
 
 MelFront::~MelFront() {
-    for (void* q : {(void*)d_window_, (void*)d_fb_, (void*)d_tw_, (void*)d_meta_, d_span_, (void*)d_fbp_})
+    for (void* q : {(void*)d_window_, (void*)d_fb_, (void*)d_tw_, (void*)d_tw512_, (void*)d_meta_, d_span_, (void*)d_fbp_})
         if (q) (void)hipFree(q);
 }
 
@@ -239,32 +468,35 @@ void MelFront::forward(const float* pcm, int B, int64_t S_stride, const int* n_s
                        int* T_out, hipStream_t s) {
     require(B > 0 && T_max >= 0 && n_samples && T_out && out, "mel: bad batch arguments");
     require(B <= 65535, "mel: at most 65535 clips per call");
-    meta_.assign((size_t)2 * B, 0);
+    meta_.assign(n_samples, n_samples + B);
     for (int b = 0; b < B; ++b) {
         require(n_samples[b] >= 0 && n_samples[b] <= S_stride, "mel: clip length outside [0, S_stride]");
         const int T = frames(n_samples[b]);
         require(T <= T_max, "mel: T_max smaller than a clip's frame count");
-        meta_[2 * (size_t)b] = n_samples[b];
-        meta_[2 * (size_t)b + 1] = T;
         T_out[b] = T;
     }
     require(pcm != nullptr || S_stride == 0 || *std::max_element(n_samples, n_samples + B) == 0,
             "mel: null pcm");
     if (T_max == 0) return;
-    if (meta_cap_ < 2 * B) {
-        if (d_meta_) PKX_HIP(hipFree(d_meta_));
-        d_meta_ = nullptr;
-        PKX_HIP(hipMalloc(&d_meta_, sizeof(int) * (size_t)2 * B));
-        meta_cap_ = 2 * B;
-    }
-    PKX_HIP(hipMemcpyAsync(d_meta_, meta_.data(), sizeof(int) * (size_t)2 * B, hipMemcpyHostToDevice, s));
     MelParams p{};
     p.pcm = pcm;
     p.S_stride = S_stride;
-    p.meta = d_meta_;
+    if (B <= MEL_INLINE_CLIPS) {
+        std::copy(meta_.begin(), meta_.end(), p.inl);   // the lengths travel with the kernel arguments
+    } else {
+        if (meta_cap_ < B) {
+            if (d_meta_) PKX_HIP(hipFree(d_meta_));
+            d_meta_ = nullptr;
+            PKX_HIP(hipMalloc(&d_meta_, sizeof(int) * (size_t)B));
+            meta_cap_ = B;
+        }
+        PKX_HIP(hipMemcpyAsync(d_meta_, meta_.data(), sizeof(int) * (size_t)B, hipMemcpyHostToDevice, s));
+        p.meta = d_meta_;
+    }
     p.window = d_window_;
     p.fb = d_fb_;
     p.tw = d_tw_;
+    p.tw512 = d_tw512_;
     p.span = (const int4*)d_span_;
     p.fb_packed = d_fbp_;
     p.fb_nnz = fb_nnz_;
@@ -279,9 +511,20 @@ void MelFront::forward(const float* pcm, int B, int64_t S_stride, const int* n_s
     p.preemph = cfg_.preemph;
     p.mag_power = cfg_.mag_power;
     p.log_guard = cfg_.log_guard;
-    launch(mel_spec_kernel, dim3(cdiv(T_max, MEL_FRAMES_PER_BLOCK), B), dim3(256), 0, s, p);
+    if (cfg_.n_fft != 512 || cfg_.mag_power != 2.0f || fb_nnz_ > MEL_FB_LDS || cfg_.n_mels > MEL_SPAN_LDS) {
+        launch(mel_spec_kernel, dim3(cdiv(T_max, MEL_FRAMES_PER_BLOCK), B), dim3(256), 0, s, p);
+    } else {
+        // four workgroups a CU (what their LDS and registers allow), each with its share of the groups
+        const int groups = cdiv(T_max, 4);
+        require((int64_t)groups * B < ((int64_t)1 << 31) - (1 << 20), "mel: too many frames for one call");
+        const int n_groups = groups * B;
+        launch(mel_spec512_kernel, dim3(std::min(n_groups, 4 * device_cu_count())), dim3(256), 0, s, p, groups, n_groups);
+    }
     PKX_LAUNCH_CHECK();
-    launch(mel_norm_kernel, dim3(cfg_.n_mels, B), dim3(256), 0, s, p);
+    const dim3 rows(cfg_.n_mels, B);
+    if (T_max <= 1024) launch(mel_norm_kernel<4>, rows, dim3(256), 0, s, p);
+    else if (T_max <= 4096) launch(mel_norm_kernel<16>, rows, dim3(256), 0, s, p);
+    else launch(mel_norm_kernel<0>, rows, dim3(256), 0, s, p);
     PKX_LAUNCH_CHECK();
     // the host copy of meta_ is reused by the next call: finish the upload first
     PKX_HIP(hipStreamSynchronize(s));

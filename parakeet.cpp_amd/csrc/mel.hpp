@@ -19,7 +19,9 @@ struct MelConfig {
 
 constexpr int MEL_MAX_NFFT = 512;       // LDS sizing of the FFT kernel
 constexpr int MEL_FRAMES_PER_BLOCK = 8;
-constexpr int MEL_FB_LDS = 2048;        // filterbank nonzeros staged in LDS (more: read from L2)
+constexpr int MEL_INLINE_CLIPS = 64;    // clip lengths passed with the kernel arguments
+constexpr int MEL_SPAN_LDS = 128;        // filters whose spans mel_spec512_kernel stages in LDS
+constexpr int MEL_FB_LDS = 640;         // filterbank nonzeros staged in LDS (more: read from L2)
 
 class MelFront {
 public:
@@ -44,7 +46,8 @@ private:
     float* d_window_ = nullptr;
     float* d_fb_ = nullptr;
     double* d_tw_ = nullptr;            // twiddles, [n_fft - 1][2]
-    int* d_meta_ = nullptr;             // per clip {samples, frames}
+    double* d_tw512_ = nullptr;         // n_fft 512: exp(-2 pi i k / 512), [512][2]
+    int* d_meta_ = nullptr;             // samples per clip (batches past MEL_INLINE_CLIPS)
     void* d_span_ = nullptr;            // int4 [n_mels]: nonzero bins of each filter, packed offset
     float* d_fbp_ = nullptr;            // packed nonzero filter values
     int fb_nnz_ = 0;

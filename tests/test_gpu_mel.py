@@ -138,3 +138,25 @@ def test_mel_on_speech_fixtures(gpu, stream, feat):
     print(f"[mel] speech max abs {err:.3e}, bit-identical {float(np.mean(got == ref)):.4f}", flush=True)
     assert err <= 1e-4
     mel.close()
+
+
+@pytest.mark.parametrize("B,n_mels,mag_power", [(70, 128, 2.0), (3, 80, 2.0), (2, 160, 2.0), (2, 80, 1.0)])
+def test_mel_frame_groups(gpu, stream, B, n_mels, mag_power):
+    """n_fft 512: the persistent frame-group kernel with more clips than travel
+    in the kernel arguments, clips that end inside a group and groups past a
+    clip's end; more filters than its LDS holds and a magnitude spectrum (the
+    general kernel)."""
+    win, fb = pm.hann_window(WIN), pm.mel_filterbank(SR, N_FFT, n_mels)
+    lens = [(7919 * (i + 1)) % 24000 + 1 for i in range(B)]
+    lens[0], lens[-1] = 24000, 255
+    pcm = _ragged(lens, seed=B)
+    print(f"[mel] B={B} n_mels={n_mels} mag_power={mag_power}", flush=True)
+    mel = gpu.Mel.create(N_FFT, WIN, HOP, n_mels, win, fb, mag_power=mag_power, per_feature=False)
+    cfg = oracle.mel_cfg(n_mels=n_mels, mag_power=mag_power, per_feature=False)
+    T_max = max(oracle.mel_frames(cfg, n) for n in lens) + 2
+    ref, T_ref = oracle.mel_batch(cfg, oracle.mel_window(win, N_FFT), fb, pcm, lens, T_max)
+    got, T = _run(gpu, stream, mel, pcm, lens, T_max)
+    assert list(T) == list(T_ref)
+    assert np.max(np.abs(got - ref)) <= 1e-5
+    assert float(np.mean(got == ref)) >= 0.99
+    mel.close()
