@@ -131,34 +131,6 @@ template <int BN> struct BLoad16<GT_F16, BN> {
     }
 };
 
-// Exact int8 -> f16 for 4 packed bytes: byte b (two's complement) becomes the
-// f16 with bit pattern 0x6400 | (b ^ 0x80) = 1024 + (b + 128); subtracting
-// 1152 leaves b exactly.  Then one correctly rounded f16 multiply by d.
-__device__ __forceinline__ void i8x4_to_f16(uint32_t w, half2v d2, half2v& lo, half2v& hi) {
-    const uint32_t u = w ^ 0x80808080u;
-    const uint32_t a = __builtin_amdgcn_perm(0x64646464u, u, 0x07010700u) ;  // [0x64,b1,0x64,b0]
-    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, u, 0x07030702u);   // [0x64,b3,0x64,b2]
-    const half2v bias = {(f16)1152.0f, (f16)1152.0f};
-    lo = (__builtin_bit_cast(half2v, a) - bias) * d2;
-    hi = (__builtin_bit_cast(half2v, b) - bias) * d2;
-}
-
-// Four 4-bit weights (nibble `hi` of each byte of w) to f16, w = s*q - m with
-// nm2 = -m: the nibble is placed in an f16 mantissa so that the half reads
-// 1024 + q (low nibble, exponent byte 0x64) or 64 + q (high nibble in mantissa
-// bits 4..7, exponent byte 0x54); subtracting 1024 or 64 is exact, then one
-// rounding in the fma.
-__device__ __forceinline__ void nib4_to_f16(uint32_t w, int hi, half2v s2, half2v nm2, half2v& lo, half2v& up) {
-    const uint32_t e = hi ? 0x54545454u : 0x64646464u;
-    const uint32_t mask = hi ? 0xFFF0FFF0u : 0xFF0FFF0Fu;
-    const f16 off = hi ? (f16)64.0f : (f16)1024.0f;
-    const half2v off2 = {off, off};
-    const uint32_t a = __builtin_amdgcn_perm(e, w, 0x07010700u) & mask;  // bytes 0, 1
-    const uint32_t b = __builtin_amdgcn_perm(e, w, 0x07030702u) & mask;  // bytes 2, 3
-    lo = (__builtin_bit_cast(half2v, a) - off2) * s2 + nm2;
-    up = (__builtin_bit_cast(half2v, b) - off2) * s2 + nm2;
-}
-
 // q8_0 device layout (slab-major): int8 q[K/64][ldw][64] and f16 d[K/64][ldw][2]; w = d*q.
 template <int BN> struct BLoad16<GT_Q8_0, BN> {
     static constexpr int NC = (BN * 4 + 255) / 256;
@@ -2761,6 +2733,7 @@ void launch_gemm(Precision prec, int wtype, int epi, const GemmParams& p, hipStr
     const bool big = (int64_t)cdiv(p.M, 128) * cdiv(p.N, 128) >= 256;
     if (dma_ok) {
         // Tile shapes from sweeps over the encoder's shapes on MI355X (M = B*T' = 2000):
+        // products of few rows run on K-split tiles (gemm_rows.hip);
         // the register-B kernels take the wide quantised products and the quantised
         // N = 1024 residual products when their grids fit one round of the chip;
         // otherwise q8_0 and q4_K weights prefer 128x128 when the grid holds >= 384 of
@@ -2770,6 +2743,7 @@ void launch_gemm(Precision prec, int wtype, int epi, const GemmParams& p, hipStr
         const int64_t t22 = (int64_t)cdiv(p.M, 128) * cdiv(p.N, 128);
         const int64_t t21 = (int64_t)cdiv(p.M, 128) * cdiv(p.N, 64);
         const bool glu = epi == EPI_GLU || epi == EPI_GLU_DW;
+        if (launch_gemm_rows(wtype, epi, p, s)) return;
         if (wtype == GT_Q8_0 && dma_rb<GT_Q8_0>(epi, p, s)) return;
         if (wtype == GT_Q4_K && dma_rb<GT_Q4_K>(epi, p, s)) return;
         if (wtype == GT_Q8_0 && dma_rb_resid<GT_Q8_0>(epi, p, s)) return;

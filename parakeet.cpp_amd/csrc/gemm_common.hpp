@@ -9,6 +9,34 @@ namespace pkx {
 // into a larger allocation keep the allocation's row count).
 __device__ __forceinline__ int slab_rows(const GemmParams& p) { return p.ldw > 0 ? p.ldw : p.N; }
 
+// Exact int8 -> f16 for 4 packed bytes: byte b (two's complement) becomes the
+// f16 with bit pattern 0x6400 | (b ^ 0x80) = 1024 + (b + 128); subtracting
+// 1152 leaves b exactly.  Then one correctly rounded f16 multiply by d.
+__device__ __forceinline__ void i8x4_to_f16(uint32_t w, half2v d2, half2v& lo, half2v& hi) {
+    const uint32_t u = w ^ 0x80808080u;
+    const uint32_t a = __builtin_amdgcn_perm(0x64646464u, u, 0x07010700u) ;  // [0x64,b1,0x64,b0]
+    const uint32_t b = __builtin_amdgcn_perm(0x64646464u, u, 0x07030702u);   // [0x64,b3,0x64,b2]
+    const half2v bias = {(f16)1152.0f, (f16)1152.0f};
+    lo = (__builtin_bit_cast(half2v, a) - bias) * d2;
+    hi = (__builtin_bit_cast(half2v, b) - bias) * d2;
+}
+
+// Four 4-bit weights (nibble `hi` of each byte of w) to f16, w = s*q - m with
+// nm2 = -m: the nibble is placed in an f16 mantissa so that the half reads
+// 1024 + q (low nibble, exponent byte 0x64) or 64 + q (high nibble in mantissa
+// bits 4..7, exponent byte 0x54); subtracting 1024 or 64 is exact, then one
+// rounding in the fma.
+__device__ __forceinline__ void nib4_to_f16(uint32_t w, int hi, half2v s2, half2v nm2, half2v& lo, half2v& up) {
+    const uint32_t e = hi ? 0x54545454u : 0x64646464u;
+    const uint32_t mask = hi ? 0xFFF0FFF0u : 0xFF0FFF0Fu;
+    const f16 off = hi ? (f16)64.0f : (f16)1024.0f;
+    const half2v off2 = {off, off};
+    const uint32_t a = __builtin_amdgcn_perm(e, w, 0x07010700u) & mask;  // bytes 0, 1
+    const uint32_t b = __builtin_amdgcn_perm(e, w, 0x07030702u) & mask;  // bytes 2, 3
+    lo = (__builtin_bit_cast(half2v, a) - off2) * s2 + nm2;
+    up = (__builtin_bit_cast(half2v, b) - off2) * s2 + nm2;
+}
+
 // 2-D XCD blocking: the nbm x nbn tile grid is cut into gm row bands x gn
 // column bands (gm * gn = 8), one rectangle per XCD, so an XCD's L2 sees only
 // its band of A rows and its band of weight columns (gn*|A| + gm*|W| bytes
@@ -72,6 +100,10 @@ __device__ __forceinline__ void epi_one(const GemmParams& p, int m, int n, float
         ((float*)p.Y)[(int64_t)m * p.ldy + n] = o > 0.f ? o : 0.f;
     }
 }
+
+// gemm_rows.hip: one f16 product of few rows on K-split tiles where that is the
+// faster kernel; false (nothing launched) where it is not.
+bool launch_gemm_rows(int wtype, int epi, const GemmParams& p, hipStream_t s);
 
 // gemm_f32.hip: one f32 product with f32 weights on K-split tiles where that is
 // the faster kernel; false (nothing launched) where it is not.

@@ -209,3 +209,32 @@ def test_linear_f32_k_split(gpu, stream, M, N, K):
     dr = gpu.DeviceArray.from_numpy(y0, stream)
     gpu.linear_residual(0, pm.GGML_F32, N, K, w, dx, M, dr, 0.5, db, stream)
     assert (np.abs(dr.numpy(stream) - (y0 + 0.5 * acc)) <= bound + 2.0 ** -22 * np.abs(y0)).all()
+
+
+@pytest.mark.parametrize("gtype", [pm.GGML_F16, pm.GGML_Q8_0, pm.GGML_Q4_K])
+@pytest.mark.parametrize("M,N,K", [(1, 32, 256), (2, 2048, 512), (17, 64, 768), (125, 1024, 4096), (130, 2048, 512),
+                                   (250, 1024, 2048), (257, 1536, 1024), (500, 1024, 1024), (129, 4096, 256),
+                                   (200, 4032, 512), (1000, 1024, 1024), (3, 96, 1280)])
+def test_linear_few_rows(gpu, stream, gtype, M, N, K):
+    """f16 path on the K-split row tiles: 16-, 32- and 64-row tiles, partial
+    row tiles, fewer and more 64-column steps than K groups; the store, and
+    the residual update twice in a row on the same inputs (bit-identical)."""
+    rng = _rng(M + 5 * N + K)
+    raw, wf = _weights(gtype, N, K, rng)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    b = rng.normal(0, 0.1, N).astype(np.float32)
+    y0 = rng.normal(0, 1, (M, N)).astype(np.float32)
+    print(f"[linear-rows] type={gtype} M={M} N={N} K={K}", flush=True)
+    ref = oracle.linear(x, wf, b)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    db = gpu.DeviceArray.from_numpy(b, stream)
+    dy = gpu.DeviceArray((M, N), np.float32)
+    gpu.linear(1, gtype, N, K, raw, dx, M, dy, db, stream)
+    assert rel_l2(dy.numpy(stream), ref) < 2e-3
+    outs = []
+    for _ in range(2):
+        dr = gpu.DeviceArray.from_numpy(y0, stream)
+        gpu.linear_residual(1, gtype, N, K, raw, dx, M, dr, 0.5, db, stream)
+        outs.append(dr.numpy(stream))
+    assert np.array_equal(outs[0], outs[1])
+    assert rel_l2(outs[0] - y0, 0.5 * ref) < 2e-3
