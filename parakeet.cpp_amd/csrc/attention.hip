@@ -86,10 +86,15 @@ __device__ __forceinline__ float xg_sum(float x) {
 // after its wait; the built code keeps the window clean (no VGPR copy or spill
 // of a transposed-load destination between the load and its s_waitcnt, read
 // from this file's gfx950 assembly).
-__device__ __forceinline__ void lds_tr_b64(half4v& r, const f16* p) {
+// lds_tr_b64_into is the same for a register that already holds a value (set
+// before the loop: no zeroing per load).
+__device__ __forceinline__ void lds_tr_b64_into(half4v& r, const f16* p) {
     const uint32_t off = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const f16*)p;
-    r = (half4v){};
     asm volatile("ds_read_b64_tr_b16 %0, %1" : "+v"(r) : "v"(off));
+}
+__device__ __forceinline__ void lds_tr_b64(half4v& r, const f16* p) {
+    r = (half4v){};
+    lds_tr_b64_into(r, p);
 }
 template <int N> __device__ __forceinline__ void lds_tr_wait(half4v& x, half4v& y) {
     static_assert(N >= 0 && N < 16, "lgkmcnt range");
@@ -449,6 +454,291 @@ __global__ __launch_bounds__(64 * NQW * NG, 1) void relpos_attn_ks_kernel(AttnPa
 }
 
 // ---------------------------------------------------------------------------
+// f16 MFMA kernel for grids past one round of the chip: 128 queries per block,
+// eight waves of 16 queries (two per SIMD), keys in steps of 64, the products
+// formed as in relpos_attn_ks_kernel.
+//
+// What bounds it is LDS bandwidth: a wave reads its step's K, band and V (52 KB
+// at DK = 128) and passes G through it, about 4.9 k cycles a step for the eight
+// waves with the bank conflicts, of the 5.6 k a step takes (MFMA 1.7 k per
+// SIMD).  The loads run a step ahead: K and V have two buffers each, and the
+// positional band is a ring of 256 rows of which a step uses 192 and the next
+// needs only 64 new ones (a third of the band's traffic), so one step's DMA is
+// 48 KB instead of 80 and has a whole step to land, behind one barrier.  Tiles
+// without a masked key skip the mask arithmetic, and the output is rescaled
+// only in steps where some query's maximum moved.  MI355X, 4 items of 3750
+// frames, 8 heads of 128: 1010 us with 96-query blocks of relpos_attn_ks_kernel
+// (four barriers a step, each load waited for in the step it was issued in),
+// 650 here.  The same waves half a step apart (one's scores under the other's
+// softmax, two barriers) 850; the second barrier with one V buffer 690.
+// ---------------------------------------------------------------------------
+template <int DK> struct LongSmem {
+    static constexpr int NW = 8, AQ = 128, RING = 256, LDG = 52;
+    f16 k[2][AK * DK];
+    f16 v[2][AK * DK];
+    f16 p[RING * DK];            // band row x (from the block's first) at x % RING
+    float g[NW][16 * LDG];       // per wave: 48 rows of G^T as [query][band row]
+};
+
+template <int DK>
+__global__ __launch_bounds__(512, 1) void relpos_attn_long_kernel(AttnParams a) {
+    static_assert(DK == 64 || DK == 128, "head dim");
+    typedef LongSmem<DK> S;
+    constexpr int AQ = S::AQ, NCH = DK / 8, NKC = DK / 32, NDT = DK / 16, PW = DK / 64;   // PW: DMA instructions a wave per 64 rows
+    __shared__ __attribute__((aligned(16))) S sm;
+    static_assert(sizeof(S) <= 160 * 1024, "LDS");
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int T = a.T, P = 2 * T - 1;
+    // work order (head, item, query block) as in relpos_attn_ks_kernel
+    const int nq = (T + AQ - 1) / AQ;
+    const int wid = xcd_tile(blockIdx.x, nq * a.B * a.H);
+    const int ib = udiv_small(wid, nq), h = udiv_small(ib, a.B);   // wid < 2^22 (checked at launch)
+    const int b = ib - h * a.B, i0 = (wid - ib * nq) * AQ;
+    const int vl = a.valid ? a.valid[b] : T;
+    const int lg = lane >> 4, lc = lane & 15;   // lane group; lane in group = this lane's query
+    const int i = i0 + 16 * w + lc;
+    const int64_t rowq = (int64_t)b * T;
+    const int nst = max((vl + AK - 1) / AK, 1);   // steps
+
+    const __amdgpu_buffer_rsrc_t rk = make_rsrc((const f16*)a.k + rowq * a.ldk + h * DK, ((int64_t)(T - 1) * a.ldk + DK) * 2);
+    const __amdgpu_buffer_rsrc_t rp = make_rsrc((const f16*)a.p + h * DK, ((int64_t)(P - 1) * a.ldp + DK) * 2);
+    const __amdgpu_buffer_rsrc_t rv = make_rsrc((const f16*)a.v + rowq * a.ldv + h * DK, ((int64_t)(T - 1) * a.ldv + DK) * 2);
+    // 64 rows from row0 into dst by DMA, 16 bytes per lane, swizzled through each
+    // lane's source chunk; rows past the end (and negative ones) arrive as zeros
+    auto dma64 = [&](__amdgpu_buffer_rsrc_t r, f16* dst, int64_t ld, int row0) {
+#pragma unroll
+        for (int u = 0; u < PW; ++u) {
+            const int ii = w + 8 * u, o = ii * 1024 + 16 * lane, rr = o / (DK * 2), t = (o % (DK * 2)) / 16;
+            const int64_t off = ((int64_t)(row0 + rr) * ld + swz(rr, t, NCH) * 8) * 2;
+            lds_dma16(r, (uint8_t*)dst + ii * 1024, off < 0 ? OOB : (uint32_t)off, 0);
+        }
+    };
+    const int rlo = T - 1 - (i0 + AQ - 1);   // the position of the block's band row 0
+    auto dma_k = [&](int st) { dma64(rk, sm.k[st & 1], a.ldk, AK * st); };
+    auto dma_v = [&](int st) { dma64(rv, sm.v[st & 1], a.ldv, AK * st); };
+    auto dma_p = [&](int x) { dma64(rp, sm.p + (x & (S::RING - 1)) * DK, a.ldp, rlo + x); };   // band rows x .. x + 63
+
+    // query rows and position biases ahead of the DMAs (vector memory returns in order)
+    half8v qu[NKC], qv[NKC];
+    {
+        half8v qx[NKC];
+        float4v bu[NKC][2], bv[NKC][2];
+#pragma unroll
+        for (int kc = 0; kc < NKC; ++kc) {
+            const int c0 = h * DK + 32 * kc + 8 * lg;
+            qx[kc] = i < T ? *(const half8v*)((const f16*)a.q + (rowq + i) * a.ldq + c0) : (half8v){};
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                bu[kc][e] = *(const float4v*)(a.bias_u + c0 + 4 * e);
+                bv[kc][e] = *(const float4v*)(a.bias_v + c0 + 4 * e);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        dma_k(0);
+#pragma unroll
+        for (int x = 0; x < 192; x += 64) dma_p(x);
+        dma_v(0);
+        // B operand of v_mfma_f32_16x16x32_f16: query lane % 16, k = 32 kc + 8 (lane / 16) + e
+#pragma unroll
+        for (int kc = 0; kc < NKC; ++kc)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float xf = (float)qx[kc][e];
+                qu[kc][e] = (f16)(xf + bu[kc][e >> 2][e & 3]);
+                qv[kc][e] = (f16)(xf + bv[kc][e >> 2][e & 3]);
+            }
+    }
+    const float sl2 = a.scale * 1.4426950408889634f;   // scores in log2 units
+    // the keys this lane's query sees: [jlo, jhi)
+    int jlo = 0, jhi = vl;
+    if (a.chunk > 0) {
+        const int qc = i / a.chunk;
+        jlo = max(0, (qc - a.left_chunks) * a.chunk);
+        jhi = min(vl, (qc + 1) * a.chunk);
+    }
+
+    float4v o[NDT];   // o[d][r] = output of query lane % 16, dim 16 d + 4 (lane / 16) + r
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) o[d] = (float4v){0.f, 0.f, 0.f, 0.f};
+    float mrow = -INFINITY, lrow = 0.f;   // running max (the same in a query's four lanes), part of the denominator
+    float* gw = sm.g[w];
+    float4v sac[4];   // S^T: sac[jt][r] = score of this lane's query, key 16 jt + 4 (lane / 16) + r
+    half4v pr[4];
+    half4v vt[NDT][2];   // transposed V: set once, then only by lds_tr_b64_into (its in-out operand)
+#pragma unroll
+    for (int d = 0; d < NDT; ++d) vt[d][0] = vt[d][1] = (half4v){};
+
+    // S^T = k . qu^T + the shifted band product: the band rows x0 .. x0 + 79 (16-row blocks that do not
+    // straddle the ring's end) times qv give G, whose rel_shift gather (bd[i][j] = G[i][15 - i + j]) is
+    // added.  G passes through the wave's own 48-row area in two halves: rows 0 .. 47 for keys 0 .. 31,
+    // rows 32 .. 79 for the others (a wave's LDS operations complete in order).
+    // Each fragment is read two groups of MFMAs before its use (groups of one 32-column k block: the
+    // band's five fragments, then K's four); left to itself the compiler reads each one MFMA ahead and
+    // the wave waits out the LDS latency 36 times a step.
+    auto scores = [&](int s) {
+        constexpr int NGR = 2 * NKC;   // groups: the band's k blocks, then K's
+        const f16* kt = sm.k[s & 1];
+        const int x0 = AK * s + AQ - 16 - 16 * w;
+        half8v fr[3][5];
+        auto fetch = [&](int g) {
+#pragma unroll
+            for (int e = 0; e < 5; ++e) {
+                if (g < NKC) {
+                    const int r = ((x0 + 16 * e) & (S::RING - 1)) + lc;
+                    fr[g % 3][e] = *(const half8v*)(sm.p + r * DK + swz(r, 4 * g + lg, NCH) * 8);
+                } else if (e < 4) {
+                    const int r = 16 * e + lc;
+                    fr[g % 3][e] = *(const half8v*)(kt + r * DK + swz(r, 4 * (g - NKC) + lg, NCH) * 8);
+                }
+            }
+        };
+        float4v gb[5];
+#pragma unroll
+        for (int gt = 0; gt < 5; ++gt) gb[gt] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt) sac[jt] = (float4v){0.f, 0.f, 0.f, 0.f};
+        float* garea = gw + lc * S::LDG + 4 * lg;
+        const float* grow = gw + lc * S::LDG + 15 - lc + 4 * lg;
+        fetch(0);
+        fetch(1);
+#pragma unroll
+        for (int g = 0; g < NGR; ++g) {
+            if (g + 2 < NGR) fetch(g + 2);
+            // G's first half leaves while K's products run
+            if (g == NKC + 1 || (NGR == 2 && g == 1)) {
+#pragma unroll
+                for (int gt = 0; gt < 3; ++gt) *(float4v*)(garea + 16 * gt) = gb[gt];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (g < NKC) {
+#pragma unroll
+                for (int e = 0; e < 5; ++e) gb[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[g % 3][e], qv[g], gb[e], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    sac[e] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[g % 3][e], qu[g - NKC], sac[e], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            if (hf == 1) {
+#pragma unroll
+                for (int gt = 0; gt < 3; ++gt) *(float4v*)(garea + 16 * gt) = gb[2 + gt];
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) sac[2 * hf + jj][r] += grow[16 * jj + r];
+            __builtin_amdgcn_wave_barrier();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // V^T fragments of 32-key block kc, dims 16 d .. + 15 (as in relpos_attn_ks_kernel)
+    auto v_read = [&](const f16* vst, int kc, int d) {
+        const int kr = 32 * kc + 4 * lg + (lc >> 2);
+        const int dc = 16 * d + 4 * (lc & 3);
+        const int r1 = kr + 16;
+        lds_tr_b64_into(vt[d][0], vst + kr * DK + swz(kr, dc / 8, NCH) * 8 + (dc & 7));
+        lds_tr_b64_into(vt[d][1], vst + r1 * DK + swz(r1, dc / 8, NCH) * 8 + (dc & 7));
+    };
+    // masks, online softmax (mrow: the running max of the scaled scores)
+    auto softmax = [&](int j0, auto MASK) {
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (decltype(MASK)::value) {
+                    const int j = j0 + 16 * jt + 4 * lg + r;
+                    sac[jt][r] += (j < jlo || j >= jhi) ? -INFINITY : 0.f;
+                }
+                tmax = fmaxf(tmax, sac[jt][r]);
+            }
+        const float mnew = fmaxf(mrow, xg_max(tmax) * sl2);   // scale > 0
+        const float msub = mnew == -INFINITY ? 0.f : mnew;   // no -inf - -inf while every key so far is masked
+        if (__any(mnew > mrow)) {   // uniform over the wave
+            const float corr = __builtin_amdgcn_exp2f(mrow - msub);
+            lrow *= corr;
+#pragma unroll
+            for (int d = 0; d < NDT; ++d) o[d] *= corr;
+            mrow = mnew;
+        }
+        float tsum = 0.f;
+#pragma unroll
+        for (int jt = 0; jt < 4; ++jt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float e = __builtin_amdgcn_exp2f(fmaf(sac[jt][r], sl2, -msub));
+                tsum += e;
+                pr[jt][r] = (f16)e;
+            }
+        lrow += tsum;
+    };
+    // O^T += v^T . prob^T.  The first block's transposed reads went out before the softmax; each MFMA's
+    // registers take the second block's as soon as it has been issued, so 2 NDT reads stay in flight.
+    auto pv = [&](const f16* vst) {
+        auto block = [&](auto KC) {
+            constexpr int kc = decltype(KC)::value;
+            const half8v pf = {pr[2 * kc][0], pr[2 * kc][1], pr[2 * kc][2], pr[2 * kc][3],
+                               pr[2 * kc + 1][0], pr[2 * kc + 1][1], pr[2 * kc + 1][2], pr[2 * kc + 1][3]};
+            auto mma = [&](auto Dc) {
+                constexpr int d = decltype(Dc)::value;
+                half4v(&x)[2] = vt[d];
+                lds_tr_wait<kc == 0 ? 2 * (NDT - 1) : 2 * (NDT - 1 - d)>(x[0], x[1]);
+                const half8v vf = {x[0][0], x[0][1], x[0][2], x[0][3], x[1][0], x[1][1], x[1][2], x[1][3]};
+                o[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pf, o[d], 0, 0, 0);
+                if constexpr (kc == 0) v_read(vst, 1, d);
+            };
+            static_for<0, NDT>(mma);
+        };
+        block(std::integral_constant<int, 0>{});
+        block(std::integral_constant<int, 1>{});
+    };
+
+    // Step s: one barrier.  Behind it every wave's share of K[s], V[s] and the
+    // band has landed and every wave is past step s - 1, so the other K and V
+    // buffers and the 64 band rows that step s - 1 was the last to use are free:
+    // step s + 1's loads go out and have this whole step to land.  Between
+    // barriers the waves drift apart, one's softmax under another's products.
+    for (int s = 0; s < nst; ++s) {
+        wait_vmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+        if (s + 1 < nst) {
+            dma_k(s + 1);
+            dma_p(192 + AK * s);
+            dma_v(s + 1);
+        }
+        const int j0 = AK * s;
+        if (j0 >= vl) continue;
+        scores(s);
+        const f16* vst = sm.v[s & 1];
+#pragma unroll
+        for (int d = 0; d < NDT; ++d) v_read(vst, 0, d);
+        if (a.chunk == 0 && j0 + AK <= vl) softmax(j0, std::false_type{});
+        else softmax(j0, std::true_type{});
+        pv(vst);
+    }
+
+    lrow = xg_sum(lrow);
+    f16* orow = (f16*)a.out + (rowq + i) * a.ldo + h * DK + 4 * lg;
+    const float inv = (i < vl && lrow > 0.f) ? 1.0f / lrow : 0.f;   // padded query rows are zero
+    if (i < T) {
+#pragma unroll
+        for (int d = 0; d < NDT; ++d) {
+            half4v hv;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) hv[r] = (f16)(o[d][r] * inv);
+            *(half4v*)(orow + 16 * d) = hv;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // f32 kernel (exact-precision path): one wave per query row, scores in LDS.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void relpos_attn_f32_kernel(AttnParams a, int dk) {
@@ -521,18 +811,28 @@ void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s)
         require(((int64_t)(2 * a.T - 2) * a.ldp + a.dk) * 2 < ((int64_t)1 << 31) &&
                     ((int64_t)(a.T + 127) * std::max(a.ldk, a.ldv) + a.dk) * 2 < ((int64_t)1 << 31),
                 "attention(f16): an item's key rows or a head's positional rows span 2 GiB or more");
-        // Blocks run one per CU (LDS).  When the last round of 64-query
-        // blocks would leave the chip partly idle, 96-query blocks of one key
-        // group (six waves, 1.5x the work each) are taken if they need
-        // fewer rounds by that measure (T' = 375 at batch 8: 384 -> 256).
+        // Blocks run one per CU (LDS).  While the 64-query blocks fit one round of the chip they
+        // are the most parallel form (0.6B attention, us, against the 128-query kernel: 1 x 375 50.6
+        // / 56.4, 8 x 200 65 / 68, 2 x 1000 88 / 100); past that the 128-query kernel's steps win
+        // (8 x 375 95.4 / 95.0, 16 x 227 103 / 100, 8 x 1000 276 / 250, 2 x 3750 575 / 455; head
+        // width 64, 110M: 8 x 375 64 / 60, 64 x 125 82 / 75, 2 x 3750 355 / 266).  Heads of 32 have no
+        // 128-query form: there, when the last round of 64-query blocks would leave the chip
+        // partly idle, 96-query blocks of one key group (six waves, 1.5x the work each) are
+        // taken if they need fewer rounds by that measure.
         const int cus = device_cu_count();
         const int64_t nb64 = (int64_t)cdiv(a.T, 64) * a.H * a.B, nb96 = (int64_t)cdiv(a.T, 96) * a.H * a.B;
+        const int64_t nb128 = (int64_t)cdiv(a.T, 128) * a.H * a.B;
         require(nb64 < ((int64_t)1 << 22), "attention(f16): more than 2^22 query blocks");
         const bool wide = 3 * ((nb96 + cus - 1) / cus) < 2 * ((nb64 + cus - 1) / cus);
         auto go = [&](auto DKc) {
             constexpr int D = decltype(DKc)::value;
-            if (wide) launch(relpos_attn_ks_kernel<D, 6, 1>, dim3(nb96), dim3(384), 0, s, a);
-            else launch(relpos_attn_ks_kernel<D, 4, 2>, dim3(nb64), dim3(512), 0, s, a);
+            if constexpr (D >= 64) {
+                if (nb64 > cus) launch(relpos_attn_long_kernel<D>, dim3(nb128), dim3(512), 0, s, a);
+                else launch(relpos_attn_ks_kernel<D, 4, 2>, dim3(nb64), dim3(512), 0, s, a);
+            } else {
+                if (wide) launch(relpos_attn_ks_kernel<D, 6, 1>, dim3(nb96), dim3(384), 0, s, a);
+                else launch(relpos_attn_ks_kernel<D, 4, 2>, dim3(nb64), dim3(512), 0, s, a);
+            }
         };
         if (a.dk == 128) go(std::integral_constant<int, 128>{});
         else if (a.dk == 64) go(std::integral_constant<int, 64>{});

@@ -226,3 +226,29 @@ def test_conformer_layer_production_shape(gpu, stream, ragged):
     assert rel_l2(got[mask] - x[mask], ref[mask] - x[mask]) < 3e-2
     assert rel_l2(got_fold[mask], ref[mask]) < 1e-2
     assert rel_l2(got_fold[mask] - x[mask], ref[mask] - x[mask]) < 3e-2
+
+
+@pytest.mark.parametrize("dk,B,T,valid", [
+    (128, 43, 130, [130, 129, 128, 127, 65, 64, 63, 1, 3, 2] + [130 - 3 * i for i in range(33)]),
+    (64, 65, 1, [1] * 65),
+    (64, 11, 330, [330, 321, 320, 257, 256, 255, 193, 192, 64, 1, 2]),
+    (128, 3, 1100, [1100, 1025, 700])])
+def test_relpos_attention_long(gpu, stream, dk, B, T, valid):
+    """More 64-query blocks than compute units: the 128-query kernel, with
+    partial query blocks and key tiles, lengths around its 64-key steps (one
+    step, the last step alone) and bands past the ring's end."""
+    H = 4
+    cfg = pm.Config(d_model=dk * H, n_layers=1, n_heads=H, ff_dim=64, n_mels=64, sub_channels=16, vocab_size=15)
+    m = pm.synthesize(cfg, "f16", heads=False, seed=dk + T)
+    gm, om = gpu.Model.from_tensors(m, gpu.PREC_F16), oracle.OracleModel(m)
+    x = np.random.default_rng(T).normal(0, 1, (B, T, dk * H)).astype(np.float32)
+    print(f"[attn-long] dk={dk} B={B} T={T}", flush=True)
+    ref = om.relpos_attention(0, x, oracle.rel_pos_encoding(T, dk * H), valid)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    dy = gpu.DeviceArray((B, T, dk * H), np.float32)
+    gm.relpos_attention(0, dx, valid, dy, stream)
+    got = dy.numpy(stream)
+    mask = _valid_mask(B, T, valid)
+    assert rel_l2(got[mask], ref[mask]) < _tol(1)
+    assert rel_l2(got[~mask], ref[~mask]) < _tol(1) if (~mask).any() else True
+    gm.close()
