@@ -639,14 +639,15 @@ void Model::finalize() {
                         std::memcpy(cat.data() + (size_t)r * 2 * P + P, whh.data() + (size_t)r * P,
                                     sizeof(float) * P);
                     }
-                    pred_.wcat[l] = upload_f32(cat);
+                    pred_.wpk[l] = upload_f32(pack_dec_weight(cat, 4 * P, 2 * P, P));
                     std::vector<float> bs((size_t)4 * P);
                     for (size_t i = 0; i < bs.size(); ++i) bs[i] = bih[i] + bhh[i];
                     pred_.bsum[l] = upload_f32(bs);
                 }
                 pred_.L = L;
-                pred_.jpred = upload_f32(*jp);   // f32 copies (dequantised) for the decode matvecs
-                pred_.jout = upload_f32(*jo);
+                // f32 copies (dequantised) for the decode products
+                pred_.jpred = upload_f32(pack_dec_weight(to_f32(*jp), Hj, P, 0));
+                pred_.jout = upload_f32(pack_dec_weight(to_f32(*jo), V, Hj, 0));
             }
         }
     }

@@ -98,14 +98,15 @@ struct HeadsDev {
 
 // RNNT/TDT prediction network on the device (prediction.hpp:27-50): the
 // stacked LSTM with each layer's [W_ih | W_hh] concatenated along K, so one
-// f32 product gives z = W_ih x + W_hh h; biases summed.
+// f32 product gives z = W_ih x + W_hh h; biases summed.  The weights are f32 in
+// the decode products' operand order (pack_dec_weight).
 struct PredDev {
     int H = 0, L = 0, V1 = 0;
     float* embed = nullptr;            // [V1][H]
-    float* wcat[4] = {};               // [4H][2H] f32 row-major
+    float* wpk[4] = {};                // [4H][2H], rows by unit then gate
     float* bsum[4] = {};               // b_ih + b_hh, [4H]
-    float* jpred = nullptr;            // joint.pred.weight as f32 [Hj][H]
-    float* jout = nullptr;             // joint.joint_net.2.weight as f32 [Vp][Hj]
+    float* jpred = nullptr;            // joint.pred.weight [Hj][H]
+    float* jout = nullptr;             // joint.joint_net.2.weight [Vp][Hj]
     bool ok() const { return L > 0; }
 };
 
@@ -138,6 +139,12 @@ enum KFam : int {
     KF_SUBSAMPLING = 0, KF_LAYERNORM, KF_GEMM_FFN, KF_GEMM_QKV, KF_GEMM_POS, KF_ATTENTION,
     KF_GEMM_OUT, KF_GEMM_PW1_GLU, KF_DWCONV, KF_GEMM_PW2, KF_POS_ENC, KF_COUNT
 };
+
+// decode.hip: [rows][K] f32 weights in the decode products' order (16-row tiles
+// of 16-column chunks); H > 0: an LSTM layer's [4H][K], gate rows of a unit side by side
+std::vector<float> pack_dec_weight(const std::vector<float>& w, int rows, int K, int H);
+struct DecodeWs;
+std::shared_ptr<DecodeWs> make_decode_ws();
 
 class Model {
 public:
@@ -270,6 +277,7 @@ private:
     DevWeight wpos_all_;   // linear_pos of all layers, [L*D][D]; layers_[l].wpos are row views
     HeadsDev heads_;
     PredDev pred_;
+    std::shared_ptr<DecodeWs> dec_ws_ = make_decode_ws();
     std::unique_ptr<Ws> ws_;
     float* conv_capture_ = nullptr;   // conformer_layer_forward's conv-module output
     struct ProfHook;

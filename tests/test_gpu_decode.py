@@ -51,6 +51,38 @@ def test_greedy_decode_matches_oracle(gpu, stream, kind, max_symbols, qtype):
     d_enc.free()
 
 
+@pytest.mark.parametrize("H,Hj,layers,vocab,B", [(20, 36, 1, 30, 1), (36, 20, 3, 43, 16), (340, 1300, 2, 2100, 33)])
+def test_greedy_decode_operand_remainders(gpu, stream, H, Hj, layers, vocab, B):
+    """Sizes that are no multiple of the products' 16-row tiles and 16-column
+    chunks, waves with no chunk and with the most (Hj above 1280), a vocabulary
+    of several argmax passes, full and started blocks of 16 items; twice, so that
+    the second call finds the first one's workspace."""
+    durations = (0, 1, 2)
+    cfg = pm.Config(d_model=64, n_layers=1, n_heads=2, ff_dim=128, n_mels=64, sub_channels=16, vocab_size=vocab,
+                    joint_hidden=Hj, pred_hidden=H, pred_rnn_layers=layers, tdt_durations=durations)
+    m = pm.add_prediction(pm.synthesize(cfg, "f32", heads=True, seed=H), seed=H)
+    for n in ("joint.joint_net.2.weight", "joint.joint_net.2.bias"):
+        t = m.tensors[n]
+        m.tensors[n] = pm.Tensor(t.gtype, t.shape, (t.data * 60.0).astype(np.float32))
+    gm = gpu.Model.from_tensors(m)
+    tr = oracle.Transducer(m)
+    rng = np.random.default_rng(B)
+    T_valid = [12] + [int(t) for t in rng.integers(0, 13, B - 1)]
+    enc = rng.standard_normal((B, 12, cfg.d_model)).astype(np.float32)
+    print(f"[decode] H={H} Hj={Hj} layers={layers} T={T_valid}", flush=True)
+    d_enc = gpu.DeviceArray.from_numpy(enc, stream)
+    want = [tr.greedy(enc[b, :T_valid[b]], durations=durations, max_symbols=3) for b in range(B)]
+    for _ in range(2):
+        got = gm.transducer_greedy(d_enc, T_valid, durations=durations, max_symbols=3, stream=stream)
+        for b in range(B):
+            for i in (0, 1, 3):
+                assert np.array_equal(got[b][i], want[b][i]), (b, i, got[b][i], want[b][i])
+            # logits below about 1e3, an f32 ulp 6e-5: two ulps move the confidence by at most 2 max|dl| p
+            assert np.max(np.abs(got[b][2] - want[b][2]), initial=0.0) <= 2.5e-4
+    assert sum(len(w[0]) for w in want) > 0
+    d_enc.free()
+
+
 def test_decode_rejects_bad_arguments(gpu, stream):
     cfg, m = _model((0, 1, 2, 3, 4))
     gm = gpu.Model.from_tensors(m)
