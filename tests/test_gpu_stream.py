@@ -202,6 +202,11 @@ VARIANTS = {
     "f32_k5": (dict(d_model=128, n_heads=4, ff_dim=256, conv_kernel=5), "f32", 0, 1e-4, 25),
     "q8_0_k5_batchnorm": (dict(d_model=256, n_heads=4, ff_dim=512, conv_kernel=5, conv_norm_type="batch_norm"),
                           "q8_0", 1, 1e-2, 25),
+    # the row-wise attention's f32 forms and more keys than its first batch of
+    # rows, the 9-tap conv with two and four channels a thread (not all in range)
+    "f32_dk64_d640": (dict(d_model=640, n_heads=10, ff_dim=256), "f32", 0, 1e-4, 25),
+    "f32_dk128_batchnorm": (dict(d_model=256, n_heads=2, ff_dim=256, conv_norm_type="batch_norm"), "f32", 0, 1e-4, 25),
+    "f16_dk128_d1152": (dict(d_model=1152, n_heads=9, ff_dim=256), "f16", 1, 1e-2, 25),
 }
 
 
