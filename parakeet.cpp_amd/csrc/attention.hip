@@ -739,7 +739,153 @@ __global__ __launch_bounds__(512, 1) void relpos_attn_long_kernel(AttnParams a) 
 }
 
 // ---------------------------------------------------------------------------
-// f32 kernel (exact-precision path): one wave per query row, scores in LDS.
+// f32 path on the matrix pipe: 16 queries a workgroup, scores [16][keys] in LDS.
+//
+// What bounds it is latency (one utterance is a few dozen workgroups): the four
+// waves split the keys into runs of 16-key tiles.  A tile's scores are
+// v_mfma_f32_16x16x4_f32 chains, keys as rows and queries as columns; k is dealt
+// so that a lane's float4 at column 16 c + 4 (lane / 16) feeds four of them.  The
+// positional term of query i and key j is row T - 1 - i + j: a key tile needs 31
+// rows, the second half of its two 16-row products being the next tile's first,
+// and takes its diagonal through 2 KB of LDS.  P.V deals the channels' 16-tiles
+// over the waves.  One wave per query (below) reads every key and positional row
+// once for each query, a row per lane; 110M, 1 x 125 frames, 8 heads of 64 on
+// MI355X: 23.0 -> 13.9 us a launch.
+// ---------------------------------------------------------------------------
+constexpr int AF_PLD = 36;   // positional scratch row, floats
+inline size_t attn_f32_mfma_lds(int T) { return sizeof(float) * 16 * ((size_t)(T + 15) / 16 * 16 + 4 + 4 * AF_PLD); }
+
+template <int DK>
+__global__ __launch_bounds__(256) void relpos_attn_f32_mfma_kernel(AttnParams a) {
+    extern __shared__ float smf[];
+    constexpr int NC = DK / 16;
+    const int T = a.T, lds = (T + 15) / 16 * 16 + 4;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const int q0 = 16 * blockIdx.x, h = blockIdx.y, b = blockIdx.z, i = q0 + lr;
+    float* sc = smf;                                        // [16][lds]
+    float* pw = smf + 16 * lds + w * 16 * AF_PLD + lr * AF_PLD;   // this lane's query row of the wave's scratch
+    const int vl = a.valid ? a.valid[b] : T;
+    const int64_t rowq = (int64_t)b * T;
+    float* out = (float*)a.out + rowq * a.ldo + h * DK;
+    const float4v zero = {0.f, 0.f, 0.f, 0.f};
+    if (q0 >= vl) {   // uniform: padded query rows are zero
+        for (int e = threadIdx.x; e < 16 * DK; e += 256)
+            if (q0 + e / DK < T) out[(int64_t)(q0 + e / DK) * a.ldo + e % DK] = 0.f;
+        return;
+    }
+    const float* k = (const float*)a.k + rowq * a.ldk + h * DK + 4 * lg;
+    const float* v = (const float*)a.v + rowq * a.ldv + h * DK;
+    const float* pp = (const float*)a.p + h * DK + 4 * lg;
+    float4v qu[NC], qv[NC];
+    {
+        const float* q = (const float*)a.q + (rowq + min(i, T - 1)) * a.ldq + h * DK + 4 * lg;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const float4v x = *(const float4v*)(q + 16 * c);
+            qu[c] = x + *(const float4v*)(a.bias_u + h * DK + 16 * c + 4 * lg);
+            qv[c] = x + *(const float4v*)(a.bias_v + h * DK + 16 * c + 4 * lg);
+        }
+    }
+    const int nt = (vl + 15) / 16, t0 = nt * w / 4, t1 = nt * (w + 1) / 4;
+    // 16 rows x 16 queries of rows . q, four partial sums
+    auto mm = [&](const float4v* x, const float4v* q) {
+        float4v s[4] = {zero, zero, zero, zero};
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[c][e], q[c][e], s[e], 0, 0, 0);
+        return (s[0] + s[1]) + (s[2] + s[3]);
+    };
+    // positional rows T - 16 - q0 + 16 m + lane % 16; those outside the band belong to padded queries or keys
+    auto load_p = [&](int m, float4v* x) {
+        const int row = max(0, min(T - 16 - q0 + 16 * m + lr, 2 * T - 2));
+#pragma unroll
+        for (int c = 0; c < NC; ++c) x[c] = *(const float4v*)(pp + (int64_t)row * a.ldp + 16 * c);
+    };
+    float4v lo = zero;
+    if (t0 < t1) {
+        float4v x[NC];
+        load_p(t0, x);
+        lo = mm(x, qv);
+    }
+    for (int t = t0; t < t1; ++t) {
+        float4v kx[NC], px[NC];
+        const float* kr = k + (int64_t)min(16 * t + lr, vl - 1) * a.ldk;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) kx[c] = *(const float4v*)(kr + 16 * c);
+        load_p(t + 1, px);
+        const float4v ac = mm(kx, qu), hi = mm(px, qv);
+        // lane: rows 4 lg + r of each product, query lr
+        __builtin_amdgcn_wave_barrier();
+        *(float4v*)(pw + 4 * lg) = lo;
+        *(float4v*)(pw + 16 + 4 * lg) = hi;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        lo = hi;
+        float4v s;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int j = 16 * t + 4 * lg + r;
+            float y = (ac[r] + pw[15 - lr + 4 * lg + r]) * a.scale;
+            if (j >= vl) y = -INFINITY;
+            if (a.chunk > 0) {
+                const int dc = i / a.chunk - j / a.chunk;
+                if (dc < 0 || dc > a.left_chunks) y = -INFINITY;   // key i itself is always seen
+            }
+            s[r] = y;
+        }
+        *(float4v*)(sc + lr * lds + 16 * t + 4 * lg) = s;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+    __syncthreads();
+    {
+        // softmax: 16 lanes a row, a wave 4 rows; rows past the valid queries may be all masked, they become zeros
+        float* r = sc + (4 * w + lg) * lds;
+        const bool live = q0 + 4 * w + lg < vl;
+        float mx = -INFINITY;
+        for (int j = lr; j < 16 * nt; j += 16) mx = fmaxf(mx, r[j]);
+#pragma unroll
+        for (int o = 1; o < 16; o *= 2) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+        float den = 0.f;
+        for (int j = lr; j < 16 * nt; j += 16) {
+            const float e = live && j < vl ? expf(r[j] - mx) : 0.f;
+            r[j] = e;
+            den += e;
+        }
+#pragma unroll
+        for (int o = 1; o < 16; o *= 2) den += __shfl_xor(den, o, 64);
+        const float inv = live ? 1.0f / den : 0.f;
+        if (lr == 0) r[lds - 4] = inv;
+    }
+    __syncthreads();
+    for (int ct = w; ct < NC; ct += 4) {
+        float4v o[4] = {zero, zero, zero, zero};
+        const float* vc = v + 16 * ct + lr;
+        for (int t = 0; t < nt; t += 4) {   // four key tiles' values in flight
+            float x[4][4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[u][e] = vc[(int64_t)min(16 * (t + u) + 4 * lg + e, vl - 1) * a.ldv];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                if (t + u >= nt) break;   // uniform
+                const float4v pr = *(const float4v*)(sc + lr * lds + 16 * (t + u) + 4 * lg);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(x[u][e], pr[e], o[e], 0, 0, 0);
+            }
+        }
+        if (i < T) {
+            const float inv = sc[lr * lds + lds - 4];
+            const float4v y = ((o[0] + o[1]) + (o[2] + o[3])) * inv;
+            *(float4v*)(out + (int64_t)i * a.ldo + 16 * ct + 4 * lg) = i < vl ? y : zero;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// f32, any head width and up to 16 K frames: one wave per query row, scores in LDS.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(64) void relpos_attn_f32_kernel(AttnParams a, int dk) {
     extern __shared__ float smf[];
@@ -841,7 +987,23 @@ void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s)
     } else {
         const size_t smem = sizeof(float) * (2 * (size_t)a.dk + (size_t)a.T);
         require(smem <= 64 * 1024, "attention(f32): T too large for the LDS score row");
-        launch(relpos_attn_f32_kernel, dim3(a.T, a.H, a.B), dim3(64), smem, s, a, a.dk);
+        // The matrix kernel where its scores fit the LDS (2400 frames), for the usual head widths and 16-byte
+        // aligned rows, from 16 frames on (110M attention module, us, one wave per query / matrix kernel: 1 x 1
+        // 31.6 / 33.7, 1 x 12 32.9 / 32.9, 1 x 125 52 / 43, 16 x 125 338 / 108, 1 x 375 191 / 74, 1 x 2000 3830 / 578).
+        auto al = [](const void* p, int64_t ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; };
+        const bool rows16 = a.T >= 16 && al(a.q, a.ldq) && al(a.k, a.ldk) && al(a.v, a.ldv) && al(a.p, a.ldp) && al(a.out, a.ldo) &&
+                            al(a.bias_u, 0) && al(a.bias_v, 0);
+        const size_t sm16 = attn_f32_mfma_lds(a.T);
+        auto go = [&](auto DKc) {
+            auto* fn = relpos_attn_f32_mfma_kernel<decltype(DKc)::value>;
+            if (sm16 > 64 * 1024)
+                PKX_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+            launch(fn, dim3(cdiv(a.T, 16), a.H, a.B), dim3(256), (uint32_t)sm16, s, a);
+        };
+        if (rows16 && sm16 <= 160 * 1024 && a.dk == 128) go(std::integral_constant<int, 128>{});
+        else if (rows16 && sm16 <= 160 * 1024 && a.dk == 64) go(std::integral_constant<int, 64>{});
+        else if (rows16 && sm16 <= 160 * 1024 && a.dk == 32) go(std::integral_constant<int, 32>{});
+        else launch(relpos_attn_f32_kernel, dim3(a.T, a.H, a.B), dim3(64), smem, s, a, a.dk);
     }
     PKX_LAUNCH_CHECK();
 }

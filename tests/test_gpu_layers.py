@@ -63,8 +63,8 @@ def _valid_mask(B, T, valid):
     return np.arange(T)[None, :] < np.asarray(valid)[:, None]
 
 
-# (16, 375): more 64-query blocks than one round of the chip holds, so the f16
-# kernel takes its 96-query single-key-group form (the 4-head cases: dk 64, 32)
+# (16, 375): more 64-query blocks than one round of the chip holds (the 4-head
+# cases): the f16 path's 128-query kernel at dk 64, 96-query blocks at dk 32
 @pytest.mark.parametrize("name", list(CASES))
 @pytest.mark.parametrize("B,T,valid", [(1, 1, [1]), (2, 37, [37, 20]), (3, 70, [70, 64, 1]),
                                        (2, 130, [130, 99]),
@@ -251,4 +251,28 @@ def test_relpos_attention_long(gpu, stream, dk, B, T, valid):
     mask = _valid_mask(B, T, valid)
     assert rel_l2(got[mask], ref[mask]) < _tol(1)
     assert rel_l2(got[~mask], ref[~mask]) < _tol(1) if (~mask).any() else True
+    gm.close()
+
+
+@pytest.mark.parametrize("dk,B,T,valid", [
+    (64, 3, 16, [16, 15, 1]), (32, 3, 17, [17, 16, 1]), (64, 1, 15, [15]), (64, 2, 125, [125, 49]), (128, 2, 66, [66, 65]),
+    (128, 1, 1100, [1050]), (64, 1, 2401, [2390]), (48, 2, 40, [40, 7])])
+def test_relpos_attention_f32_tiles(gpu, stream, dk, B, T, valid):
+    """The f32 matrix kernel's 16-query and 16-key tiles: one tile, waves with no
+    tile, lengths on and beside a tile's edge, scores beyond 64 KB of LDS; and the
+    row kernel below 16 frames, past the scores' limit and for another head width."""
+    H = 2
+    cfg = pm.Config(d_model=dk * H, n_layers=1, n_heads=H, ff_dim=64, n_mels=64, sub_channels=16, vocab_size=15)
+    m = pm.synthesize(cfg, "f32", heads=False, seed=dk + T)
+    gm, om = gpu.Model.from_tensors(m, gpu.PREC_F32), oracle.OracleModel(m)
+    x = np.random.default_rng(T).normal(0, 1, (B, T, dk * H)).astype(np.float32)
+    print(f"[attn-f32] dk={dk} B={B} T={T}", flush=True)
+    ref = om.relpos_attention(0, x, oracle.rel_pos_encoding(T, dk * H), valid)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    dy = gpu.DeviceArray((B, T, dk * H), np.float32)
+    gm.relpos_attention(0, dx, valid, dy, stream)
+    got = dy.numpy(stream)
+    mask = _valid_mask(B, T, valid)
+    assert rel_l2(got[mask], ref[mask]) < _tol(0)
+    assert rel_l2(got[~mask], ref[~mask]) < _tol(0) if (~mask).any() else True
     gm.close()
