@@ -2505,8 +2505,7 @@ static void dma_22q(int epi, const GemmParams& p, hipStream_t s) {
     }
 }
 // Split-K across workgroups for the residual products of few rows and K >= 1024
-// (a streaming step's FFN linear2: M = streams x chunk frames, 64 x 64 tiles in
-// the tens): 64 x 64 tiles in two K groups, the K range cut over S workgroups
+// that the K-split tiles do not take (N no multiple of 32, unaligned operands): 64 x 64 tiles in two K groups, the K range cut over S workgroups
 // per tile (S a power of two up to 8, each K group keeping at least one 64-deep
 // slab) until the grid holds about one workgroup per CU.  On MI355X at M = 512,
 // N = 512, K = 2048: 64 tiles x 4 splits, 1.4 us faster per launch; at K = 512
