@@ -256,8 +256,8 @@ int pkx_rel_pos_encoding(int T, int D, float* out_dev, void* stream);
  * enc_dev [B][T_max][d_model] f32 (the encoder output, time-major), T_valid
  * (host) frames per item.  Outputs (host, [B][cap] each, NULL to skip): token
  * ids, NeMo frame / max_prob confidence / span per token (src/decode_types.hpp);
- * counts (host) [B] tokens per item.  A decode needing more than cap tokens
- * for an item is an error. */
+ * counts (host) [B] tokens per item; the entries past an item's tokens are 0.
+ * A decode needing more than cap tokens for an item is an error. */
 int pkx_transducer_greedy(pkx_model* m, const float* enc_dev, int B, int T_max, const int* T_valid,
                           const int32_t* durations, int n_durations, int blank_id, int max_symbols, int cap,
                           int32_t* ids, int32_t* frames, float* conf, int32_t* span, int* counts, void* stream);

@@ -410,7 +410,9 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
     int32_t *d_dur, *d_ids, *d_fr, *d_sp;
     // ints: t [0, B), active [B, 2B), sym [2B, 3B), count [3B, 4B), T [5B, 6B), overflow 6B
     const size_t n_ints = (size_t)6 * B + 1;
-    char* zero0 = nullptr;   // the operands (zero beyond what is written) and the cell states start as zeros
+    // the operands (zero beyond what is written), the cell states and the token records (their whole
+    // [B][cap] is copied out, and an earlier call's records may lie here) start as zeros
+    char* zero0 = nullptr;
     size_t zero_bytes = 0;
     auto carve = [&](char* base) {
         Carve m{base};
@@ -423,6 +425,10 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
         }
         g = m.get<float>((size_t)B16 * gc * 16);
         f = m.get<float>((size_t)B16 * fc * 16);
+        d_ids = m.get<int32_t>((size_t)B * cap);
+        d_fr = m.get<int32_t>((size_t)B * cap);
+        d_sp = m.get<int32_t>((size_t)B * cap);
+        d_cf = m.get<float>((size_t)B * cap);
         zero0 = base + z0;
         zero_bytes = m.at - z0;
         for (int l = 0; l < L; ++l) {
@@ -430,10 +436,6 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
             oc[l] = m.get<float>((size_t)B * H);
         }
         lg = m.get<float>((size_t)B * Vp);
-        d_ids = m.get<int32_t>((size_t)B * cap);
-        d_fr = m.get<int32_t>((size_t)B * cap);
-        d_sp = m.get<int32_t>((size_t)B * cap);
-        d_cf = m.get<float>((size_t)B * cap);
         ep = m.get<float>((size_t)B * T_max * Hj);
         return m.at;
     };
@@ -462,7 +464,7 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
     std::copy(durations, durations + n_dur, h_dur);
     PKX_HIP(hipMemcpyAsync(ints, h, sizeof(int) * n_ints, hipMemcpyHostToDevice, s));
     if (n_dur > 0) PKX_HIP(hipMemcpyAsync(d_dur, h_dur, sizeof(int32_t) * n_dur, hipMemcpyHostToDevice, s));
-    PKX_HIP(hipMemsetAsync(zero0, 0, zero_bytes, s));   // SOS input, zero state
+    PKX_HIP(hipMemsetAsync(zero0, 0, zero_bytes, s));   // SOS input, zero state, no records
     DecState st{ints, ints + B, ints + 2 * B, ints + 3 * B, ints + 6 * B, ints + 5 * B};
 
     // enc_proj over every frame of every item (joint.cpp:37-63)

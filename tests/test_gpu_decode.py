@@ -4,6 +4,8 @@ transducer_batch.cpp reproduces in lockstep).  Bar: identical token ids,
 frames and spans per item (the argmax decisions), confidence within 1e-5.
 The joint's output weights are scaled up so that the decisions have margins
 far above f32 rounding (the device sums the products in another order)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -160,3 +162,37 @@ def test_greedy_decode_production_shape(gpu, stream):
     assert total > 100
     d_enc.free()
     gm.close()
+
+
+def _raw_greedy(gpu, gm, d_enc, T_valid, durations, blank, cap, stream):
+    """pkx_transducer_greedy into arrays of -7: (ids, frames, conf, span) as [B][cap] and the counts."""
+    B, T_max, _ = d_enc.shape
+    ids, fr, sp = (np.full((B, cap), -7, np.int32) for _ in range(3))
+    cf, cnt = np.full((B, cap), -7, np.float32), np.zeros(B, np.int32)
+    tv, du = np.asarray(T_valid, np.int32), np.asarray(durations, np.int32)
+    i32, f32 = C.POINTER(C.c_int32), C.POINTER(C.c_float)
+    gpu.check(gpu.lib().pkx_transducer_greedy(
+        gm.handle, d_enc.ptr, B, T_max, tv.ctypes.data_as(i32), du.ctypes.data_as(i32), len(du), blank, 10, cap,
+        ids.ctypes.data_as(i32), fr.ctypes.data_as(i32), cf.ctypes.data_as(f32), sp.ctypes.data_as(i32),
+        cnt.ctypes.data_as(i32), stream.handle))
+    return (ids, fr, cf, sp), cnt
+
+
+def test_greedy_decode_leaves_no_earlier_tokens(gpu, stream):
+    """The outputs past an item's tokens are zeros, also after a call with more
+    tokens whose records lay at the same place of the model's workspace."""
+    durations = (0, 1, 2, 3, 4)
+    cfg, m = _model(durations)
+    gm = gpu.Model.from_tensors(m)
+    enc = np.random.default_rng(5).standard_normal((3, 40, cfg.d_model)).astype(np.float32)
+    d_enc = gpu.DeviceArray.from_numpy(enc, stream)
+    most = None
+    for T_valid in ([40, 40, 40], [3, 0, 11]):
+        print(f"[decode] T={T_valid}", flush=True)
+        out, cnt = _raw_greedy(gpu, gm, d_enc, T_valid, durations, cfg.vocab_size, 400, stream)
+        for b in range(3):
+            for a in out:
+                assert not a[b, cnt[b]:].any(), (T_valid, b, cnt[b], a[b, cnt[b]:cnt[b] + 8])
+        most = cnt if most is None else most
+    assert (cnt < most).all()
+    d_enc.free()
