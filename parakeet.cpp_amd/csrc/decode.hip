@@ -537,9 +537,12 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
     // tokens per frame: (max_symbols + 1) rounds per frame bound the loop.
     // Chunk i's flags are read while chunk i + 1 runs: no gap at a chunk's end, for
     // one chunk of rounds that change nothing (16 items of 125 frames, 0.6B decoder,
-    // with the kernels above: 7.1 -> 3.6 ms a call).
+    // with the kernels above: 7.1 -> 3.6 ms a call).  Those rounds are a short call's
+    // cost: with chunks of 8 one item of 12 frames took 522 us (497 with a wait after
+    // each chunk and no look-ahead), with 4 453; 375 frames 10.1 and 10.2 ms.  Two
+    // rounds no longer cover the host's launches (11.3).
     const int64_t max_rounds = (int64_t)T_max * (max_symbols + 1) + 1;
-    constexpr int CHUNK = 8;
+    constexpr int CHUNK = 4;
     int64_t rounds = 0;
     for (int i = 0;; ++i) {
         for (int r = 0; r < CHUNK; ++r) round();
