@@ -957,23 +957,29 @@ void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s)
         require(((int64_t)(2 * a.T - 2) * a.ldp + a.dk) * 2 < ((int64_t)1 << 31) &&
                     ((int64_t)(a.T + 127) * std::max(a.ldk, a.ldv) + a.dk) * 2 < ((int64_t)1 << 31),
                 "attention(f16): an item's key rows or a head's positional rows span 2 GiB or more");
-        // Blocks run one per CU (LDS).  While the 64-query blocks fit one round of the chip they
-        // are the most parallel form (0.6B attention, us, against the 128-query kernel: 1 x 375 50.6
-        // / 56.4, 8 x 200 65 / 68, 2 x 1000 88 / 100); past that the 128-query kernel's steps win
-        // (8 x 375 95.4 / 95.0, 16 x 227 103 / 100, 8 x 1000 276 / 250, 2 x 3750 575 / 455; head
-        // width 64, 110M: 8 x 375 64 / 60, 64 x 125 82 / 75, 2 x 3750 355 / 266).  Heads of 32 have no
-        // 128-query form: there, when the last round of 64-query blocks would leave the chip
-        // partly idle, 96-query blocks of one key group (six waves, 1.5x the work each) are
-        // taken if they need fewer rounds by that measure.
+        // Blocks run one per CU (LDS), so a grid takes whole rounds of the chip, a 128-query block's
+        // round being the longer one: heads of 64 and 128 take 128-query blocks where those need fewer
+        // rounds (us, 64 / 128 queries a block; 0.6B attention module 8 x 375 95.4 / 95.0, 16 x 227
+        // 103 / 100, 8 x 1000 276 / 250, 2 x 3750 575 / 455; 110M 64 x 125 82 / 75, 2 x 3750 355 / 266) and
+        // 64-query blocks where not (0.6B module 1 x 375 50.6 / 56.4; the kernel alone, 8 heads of 128:
+        // 11 x 257 26.8 / 30.3; 4 of 128: 40 x 160 20.7 / 24.7; 4 of 64: 40 x 160 15.5 / 16.6).  Items of at most
+        // 64 frames are one block either way: the 128-query kernel's smaller step wins at heads of 64
+        // (kernel, 8 heads: 33 x 32 9.3 / 8.3, 64 x 64 10.6 / 9.0) and at 128 only past 56 frames (33 x 16
+        // 10.8 / 11.6, 33 x 48 12.3 / 12.6, 33 x 56 12.9 / 13.0, 33 x 64 13.3 / 12.7).  Heads of 32 have no
+        // 128-query form: there, when the last round of 64-query blocks would leave the chip partly
+        // idle, 96-query blocks of one key group (six waves, 1.5x the work each) are taken if they
+        // need fewer rounds by that measure.
         const int cus = device_cu_count();
         const int64_t nb64 = (int64_t)cdiv(a.T, 64) * a.H * a.B, nb96 = (int64_t)cdiv(a.T, 96) * a.H * a.B;
         const int64_t nb128 = (int64_t)cdiv(a.T, 128) * a.H * a.B;
         require(nb64 < ((int64_t)1 << 22), "attention(f16): more than 2^22 query blocks");
-        const bool wide = 3 * ((nb96 + cus - 1) / cus) < 2 * ((nb64 + cus - 1) / cus);
+        const int r64 = cdiv(nb64, cus);
+        const bool wide = 3 * cdiv(nb96, cus) < 2 * r64;
+        const bool q128 = cdiv(nb128, cus) < r64 || (r64 > 1 && a.T <= 64 && (a.dk == 64 || a.T > 56));
         auto go = [&](auto DKc) {
             constexpr int D = decltype(DKc)::value;
             if constexpr (D >= 64) {
-                if (nb64 > cus) launch(relpos_attn_long_kernel<D>, dim3(nb128), dim3(512), 0, s, a);
+                if (q128) launch(relpos_attn_long_kernel<D>, dim3(nb128), dim3(512), 0, s, a);
                 else launch(relpos_attn_ks_kernel<D, 4, 2>, dim3(nb64), dim3(512), 0, s, a);
             } else {
                 if (wide) launch(relpos_attn_ks_kernel<D, 6, 1>, dim3(nb96), dim3(384), 0, s, a);

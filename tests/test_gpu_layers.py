@@ -232,11 +232,17 @@ def test_conformer_layer_production_shape(gpu, stream, ragged):
     (128, 43, 130, [130, 129, 128, 127, 65, 64, 63, 1, 3, 2] + [130 - 3 * i for i in range(33)]),
     (64, 65, 1, [1] * 65),
     (64, 11, 330, [330, 321, 320, 257, 256, 255, 193, 192, 64, 1, 2]),
-    (128, 3, 1100, [1100, 1025, 700])])
+    (128, 4, 1100, [1100, 1025, 700, 640]),
+    (128, 65, 57, [57, 56, 1] + [57 - (i % 50) for i in range(62)]),
+    # as many rounds with 128-query blocks, or items of one short block: 64-query blocks on several rounds
+    (128, 40, 160, [160, 129, 128, 65, 1] + [160 - 4 * i for i in range(35)]),
+    (64, 40, 129, [129, 128, 64, 1] + [129 - 3 * i for i in range(36)]),
+    (128, 65, 56, [56, 55, 1] + [56 - (i % 50) for i in range(62)])])
 def test_relpos_attention_long(gpu, stream, dk, B, T, valid):
     """More 64-query blocks than compute units: the 128-query kernel, with
     partial query blocks and key tiles, lengths around its 64-key steps (one
-    step, the last step alone) and bands past the ring's end."""
+    step, the last step alone) and bands past the ring's end; and the sizes on
+    the other side of its rule."""
     H = 4
     cfg = pm.Config(d_model=dk * H, n_layers=1, n_heads=H, ff_dim=64, n_mels=64, sub_channels=16, vocab_size=15)
     m = pm.synthesize(cfg, "f16", heads=False, seed=dk + T)
