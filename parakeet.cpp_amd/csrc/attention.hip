@@ -994,10 +994,14 @@ void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s)
         const size_t smem = sizeof(float) * (2 * (size_t)a.dk + (size_t)a.T);
         require(smem <= 64 * 1024, "attention(f32): T too large for the LDS score row");
         // The matrix kernel where its scores fit the LDS (2400 frames), for the usual head widths and 16-byte
-        // aligned rows, from 16 frames on (110M attention module, us, one wave per query / matrix kernel: 1 x 1
-        // 31.6 / 33.7, 1 x 12 32.9 / 32.9, 1 x 125 52 / 43, 16 x 125 338 / 108, 1 x 375 191 / 74, 1 x 2000 3830 / 578).
+        // aligned rows, from 64 frames on, or from 16 where the other kernel's waves (one per query and
+        // head) are more than four per CU (kernel alone, us, one wave per query / matrix kernel: heads of
+        // 128, 8 x 1 x 16 6.9 / 8.1, 8 x 1 x 48 9.8 / 9.8, 8 x 1 x 64 12.0 / 11.0; of 64, 4 x 1 x 17 5.3 / 5.9, 4 x 16 x 17
+        // 6.5 / 6.0, 4 x 1 x 64 7.3 / 7.3; of 32, 4 x 4 x 17 4.8 / 5.1, 4 x 16 x 17 5.4 / 5.1 (heads x items x frames);
+        // 110M attention module: 1 x 125 52 / 43, 16 x 125 338 / 108, 1 x 375 191 / 74, 1 x 2000 3830 / 578).
         auto al = [](const void* p, int64_t ld) { return (uintptr_t)p % 16 == 0 && ld % 4 == 0; };
-        const bool rows16 = a.T >= 16 && al(a.q, a.ldq) && al(a.k, a.ldk) && al(a.v, a.ldv) && al(a.p, a.ldp) && al(a.out, a.ldo) &&
+        const bool fill = a.T >= 64 || (a.T >= 16 && (int64_t)a.T * a.H * a.B > 4 * (int64_t)device_cu_count());
+        const bool rows16 = fill && al(a.q, a.ldq) && al(a.k, a.ldk) && al(a.v, a.ldv) && al(a.p, a.ldp) && al(a.out, a.ldo) &&
                             al(a.bias_u, 0) && al(a.bias_v, 0);
         const size_t sm16 = attn_f32_mfma_lds(a.T);
         auto go = [&](auto DKc) {

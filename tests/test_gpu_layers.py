@@ -261,12 +261,14 @@ def test_relpos_attention_long(gpu, stream, dk, B, T, valid):
 
 
 @pytest.mark.parametrize("dk,B,T,valid", [
-    (64, 3, 16, [16, 15, 1]), (32, 3, 17, [17, 16, 1]), (64, 1, 15, [15]), (64, 2, 125, [125, 49]), (128, 2, 66, [66, 65]),
-    (128, 1, 1100, [1050]), (64, 1, 2401, [2390]), (48, 2, 40, [40, 7])])
+    (64, 33, 16, [16, 15, 1] + [16 - i % 16 for i in range(30)]), (32, 31, 17, [17, 16, 1] + [17 - i % 17 for i in range(28)]),
+    (128, 2, 64, [64, 49]), (64, 2, 125, [125, 49]), (128, 2, 66, [66, 65]), (128, 1, 1100, [1050]),
+    (64, 3, 16, [16, 15, 1]), (32, 3, 17, [17, 16, 1]), (128, 3, 63, [63, 17, 1]), (64, 1, 15, [15]), (64, 1, 2401, [2390]), (48, 2, 40, [40, 7])])
 def test_relpos_attention_f32_tiles(gpu, stream, dk, B, T, valid):
     """The f32 matrix kernel's 16-query and 16-key tiles: one tile, waves with no
     tile, lengths on and beside a tile's edge, scores beyond 64 KB of LDS; and the
-    row kernel below 16 frames, past the scores' limit and for another head width."""
+    row kernel on the other side of the rule (below 64 frames at few items, below
+    16, past the scores' limit, another head width)."""
     H = 2
     cfg = pm.Config(d_model=dk * H, n_layers=1, n_heads=H, ff_dim=64, n_mels=64, sub_channels=16, vocab_size=15)
     m = pm.synthesize(cfg, "f32", heads=False, seed=dk + T)
