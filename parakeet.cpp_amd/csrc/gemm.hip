@@ -2781,13 +2781,19 @@ void launch_gemm(Precision prec, int wtype, int epi, const GemmParams& p, hipStr
         }
     } else {
         if (wtype == GT_F32 && launch_gemm_f32_ks(epi, p, s)) return;
-        // 64x128 tiles when their last round of the chip is at least 90% full (M = 2000,
-        // N = 2048, K = 512: 512 tiles 51.6 us against 56.2 with 32x64; N = 1025, K = 1024: 288
-        // tiles, a second round for 32 of them, 86.6 against 61.9), else 32x64 while those
-        // fill the chip, else 32x32
-        const int64_t t24 = (int64_t)cdiv(p.M, 64) * cdiv(p.N, 128), cus = device_cu_count();
+        // 64x128 tiles when their last round of the chip is full enough, else 32x64 (GLU 32x128) while those
+        // fill the chip, else 32x32.  The last round pays, at one to two rounds, from half of it on for GLU
+        // (whose 32x128 tiles then need a fourth half round) and for quantised weights (dequantised once
+        // more for every row of tiles), else from three quarters; past two rounds at 90% over all (us,
+        // 64x128 / smaller tiles; q8_0 N = 3072, K = 1024: M = 827, 1.2 rounds, 85 / 62, M = 1019, 1.5, 86 / 93,
+        // M = 1211, 1.8, 91 / 98, M = 1531, 2.25, 173 / 117, M = 2235, 3.3, 179 / 165; GLU q8_0 N = 3072, K = 512: M =
+        // 1019 45 / 38, M = 1083, 1.6 rounds, 45 / 52; f16 N = 1536, K = 1024: M = 2235, 1.6 rounds, 84 / 79, M =
+        // 2427, 1.8, 84 / 88; f32 N = 1024, K = 512: M = 3387, 1.7, 46.7 / 46.0, M = 3643, 1.8, 46.8 / 48.2)
+        const int64_t t24 = (int64_t)cdiv(p.M, 64) * cdiv(p.N, 128), cus = device_cu_count(), rounds = cdiv(t24, cus);
         const int64_t t12 = (int64_t)cdiv(p.M, 32) * cdiv(p.N, 64);
-        const int shape = t24 >= 256 && 10 * t24 >= 9 * cus * cdiv(t24, cus) ? 0 : t12 >= 256 ? 1 : 2;
+        // the line in fortieths of a round (GLU: just past the half, where three half rounds still win)
+        const int64_t line = rounds != 2 ? 36 * rounds : epi == EPI_GLU ? 61 : wtype == GT_Q8_0 || wtype == GT_Q4_K ? 60 : 70;
+        const int shape = t24 >= 256 && 40 * t24 >= line * cus ? 0 : t12 >= 256 ? 1 : 2;
         switch (wtype) {
         case GT_F32: f32_shape<GT_F32>(shape, epi, p, s); break;
         case GT_F16: f32_shape<GT_F16>(shape, epi, p, s); break;

@@ -211,6 +211,26 @@ def test_linear_f32_k_split(gpu, stream, M, N, K):
     assert (np.abs(dr.numpy(stream) - (y0 + 0.5 * acc)) <= bound + 2.0 ** -22 * np.abs(y0)).all()
 
 
+@pytest.mark.parametrize("gtype", [pm.GGML_F32, pm.GGML_F16, pm.GGML_Q8_0, pm.GGML_Q4_K])
+@pytest.mark.parametrize("M", [827, 1019, 1147, 1211, 1403, 1787])
+def test_linear_f32_mode_tiles(gpu, stream, gtype, M):
+    """f32 mode past one round of 64 x 128 tiles (N = 3072): 1.2 to 1.8 rounds,
+    where the 64 x 128 and the 32 x 64 tiles alternate by weight type, and 2.1
+    and 2.6."""
+    N, K = 3072, 256
+    rng = _rng(M)
+    raw, wf = _weights(gtype, N, K, rng)
+    x = rng.normal(0, 1, (M, K)).astype(np.float32)
+    b = rng.normal(0, 0.1, N).astype(np.float32)
+    print(f"[linear-f32-tiles] type={gtype} M={M}", flush=True)
+    ref = oracle.linear(x, wf, b)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    db = gpu.DeviceArray.from_numpy(b, stream)
+    dy = gpu.DeviceArray((M, N), np.float32)
+    gpu.linear(0, gtype, N, K, raw, dx, M, dy, db, stream)
+    assert rel_l2(dy.numpy(stream), ref) < 1e-5
+
+
 @pytest.mark.parametrize("gtype", [pm.GGML_F16, pm.GGML_Q8_0, pm.GGML_Q4_K])
 @pytest.mark.parametrize("M,N,K", [(1, 32, 256), (2, 2048, 512), (17, 64, 768), (125, 1024, 4096), (130, 2048, 512),
                                    (250, 1024, 2048), (257, 1536, 1024), (500, 1024, 1024), (129, 4096, 256),

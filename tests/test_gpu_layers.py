@@ -118,6 +118,25 @@ def test_conv_module_item_tiles(gpu, stream, name, B, T, valid):
     test_conv_module(gpu, stream, name, B, T, valid)
 
 
+@pytest.mark.parametrize("wt", ["f32", "f16"])
+@pytest.mark.parametrize("B,T,valid", [(3, 1500, [1500, 1499, 3]), (3, 2000, [2000, 64, 1999]), (3, 2100, [2100, 2099, 1]),
+                                       (5, 1700, [1700, 1, 33, 1699, 64])])
+def test_conv_module_f32_glu_tiles(gpu, stream, wt, B, T, valid):
+    """pointwise_conv1 + GLU in f32 mode (N = 512) where its tiles change: one
+    round of 64 x 128 tiles, one and a half, just past that and two."""
+    m = pm.synthesize(_cfg(dict(d_model=256, n_heads=4, ff_dim=64), n_layers=1), wt, bn_random=True)
+    om, gm = oracle.OracleModel(m), gpu.Model.from_tensors(m, gpu.PREC_F32)
+    c = np.random.default_rng(T).normal(0, 1, (B, T, 256)).astype(np.float32)
+    print(f"[conv-f32] {wt} B={B} T={T}", flush=True)
+    ref = om.conv_module(0, c, valid)
+    dc = gpu.DeviceArray.from_numpy(c, stream)
+    dy = gpu.DeviceArray((B, T, 256), np.float32)
+    gm.conv_module(0, dc, valid, dy, stream)
+    mask = _valid_mask(B, T, valid)
+    assert rel_l2(dy.numpy(stream)[mask], ref[mask]) < _tol(0)
+    gm.close()
+
+
 @pytest.mark.parametrize("name", list(CASES) + ["q8_d512", "f16_d512"])
 @pytest.mark.parametrize("B,T,valid", [(1, 26, [26]), (2, 63, [63, 40])])
 def test_conformer_layer(gpu, stream, name, B, T, valid):
