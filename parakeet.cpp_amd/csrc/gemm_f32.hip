@@ -218,6 +218,10 @@ bool launch_gemm_f32_ks(int epi, const GemmParams& p, hipStream_t s) {
     if (epi == EPI_GLU_DW || epi == EPI_RESID_LN) return false;
     // the DMA's 16-byte pieces, and row offsets within a tile below 2 GB
     if (((uintptr_t)p.A | (uintptr_t)p.Wq) & 15 || p.lda % 4 || p.K > (1 << 20) || p.lda > (1 << 20)) return false;
+    // short K leaves nothing to split: the other kernel is faster, but for GLU, which costs it 128-column
+    // tiles (K = 128: M = 1000, N = 128 4.3 against 5.0, M = 2, N = 1025 3.9 against 4.4; GLU M = 125, N = 256 7.8
+    // against 4.6)
+    if (p.K < 256 && epi != EPI_GLU) return false;
     const int64_t t12 = (int64_t)cdiv(p.M, 16) * cdiv(p.N, 32), t22 = (int64_t)cdiv(p.M, 32) * cdiv(p.N, 32);
     const int cus = device_cu_count();
     if (t12 <= cus) {
@@ -236,10 +240,11 @@ bool launch_gemm_f32_ks(int epi, const GemmParams& p, hipStream_t s) {
         run_f32_ks<2, 2, 4, 2>(epi, p, s);
         return true;
     }
-    // GLU: the barrier-per-slab kernel needs 128-column tiles; single-wave 32 x 32 tiles
-    // with five co-resident per CU beat them (K = 512, N = 1024: M = 1000 15.7 against
-    // 19.5, M = 2000 25.2 against 29.2; not measured past sixteen tiles per CU)
-    if (epi == EPI_GLU && t22 <= 16 * cus) {
+    // GLU: the barrier-per-slab kernel needs 128-column tiles; single-wave 32 x 32 tiles with five
+    // co-resident per CU beat them up to nine tiles per CU, about one round of its tiles (K = 512,
+    // N = 1024: M = 1000 15.7 against 19.5, M = 2000 23.0 against 29.1, M = 2250 31.2 against 37.6; M = 2500,
+    // 9.9 tiles, 41.6 against 37.8, M = 4000 51.7 against 47.0)
+    if (epi == EPI_GLU && t22 <= 9 * cus) {
         run_f32_ks<2, 2, 1, 2>(epi, p, s);
         return true;
     }

@@ -186,11 +186,11 @@ def test_residual_two_k_groups(gpu, stream, gtype, K):
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 33, 8), (17, 31, 1000), (125, 512, 2048), (16, 32, 1024), (249, 2048, 520),
-                                   (33, 1025, 40), (1000, 1030, 1032), (700, 512, 512), (513, 640, 1024)])
+                                   (33, 1025, 40), (33, 1025, 264), (1, 31, 256), (1000, 1030, 1032), (700, 512, 512), (513, 640, 1024)])
 def test_linear_f32_k_split(gpu, stream, M, N, K):
     """f32 weights on the K-split tiles (16 x 32 with four and eight K groups,
     32 x 32 with four): partial tiles on both edges, K that is no whole number
-    of 32-column steps, fewer steps than K groups.  Every element within the
+    of 32-column steps; and K below the K-split kernel's 256.  Every element within the
     worst-case f32 summation bound of the float64 product, for the store and
     for the residual update."""
     rng = _rng(M + 3 * N + K)
