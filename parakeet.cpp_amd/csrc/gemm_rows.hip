@@ -374,8 +374,11 @@ static bool rows_shape(int epi, const GemmParams& p, hipStream_t s) {
         return true;
     }
     // quantised: three 32-row tiles per CU (M = 250, N = 3072, K = 1024: 8.8 against 10.2; four,
-    // N = 4096: 11.1 against 10.8; f16 weights at three, M = 749, N = 1024: 9.9 against 8.9)
-    if (WT != GT_F16 && t2 <= 3 * cus) {
+    // N = 4096: 11.1 against 10.8; f16 weights at three, M = 749, N = 1024: 9.9 against 8.9), two where
+    // K is below 512 (K = 256: M = 96, N = 4352 1.6 per CU, 10% faster, M = 640, N = 1024, 2.5, 5.7 against 5.3; GLU
+    // gains at three too)
+    const int64_t per_cu = p.K >= 512 || epi == EPI_GLU ? 3 : 2;
+    if (WT != GT_F16 && t2 <= per_cu * cus) {
         run_rows<2, 4, 2, WT>(epi, p, s);
         return true;
     }

@@ -234,7 +234,7 @@ def test_linear_f32_mode_tiles(gpu, stream, gtype, M):
 @pytest.mark.parametrize("gtype", [pm.GGML_F16, pm.GGML_Q8_0, pm.GGML_Q4_K])
 @pytest.mark.parametrize("M,N,K", [(1, 32, 256), (2, 2048, 512), (17, 64, 768), (125, 1024, 4096), (130, 2048, 512),
                                    (250, 1024, 2048), (257, 1536, 1024), (500, 1024, 1024), (129, 4096, 256),
-                                   (200, 4032, 512), (1000, 1024, 1024), (3, 96, 1280)])
+                                   (129, 3072, 256), (200, 4032, 512), (1000, 1024, 1024), (3, 96, 1280)])
 def test_linear_few_rows(gpu, stream, gtype, M, N, K):
     """f16 path on the K-split row tiles: 16-, 32- and 64-row tiles, partial
     row tiles, fewer and more 64-column steps than K groups; the store, and
