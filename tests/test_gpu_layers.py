@@ -118,6 +118,28 @@ def test_conv_module_item_tiles(gpu, stream, name, B, T, valid):
     test_conv_module(gpu, stream, name, B, T, valid)
 
 
+@pytest.mark.parametrize("name", ["q8_dk64", "q4k_dk128", "f16_k5"])
+@pytest.mark.parametrize("B,T,valid", [(3, 250, [250, 249, 7]), (5, 300, [300, 1, 299, 64, 65])])
+def test_conformer_layer_few_row_tiles(gpu, stream, name, B, T, valid):
+    """A block whose products fall on the few-row kernel's larger tiles: SiLU of
+    quantised weights (N = 512) on 64 rows at 750 frames; GLU as a product of its
+    own (five-tap conv, N = 256, LayerNorm folded in) on 32 rows at 750 and on 64
+    at 1500.  The conv module alone runs the GLU without the folding."""
+    m, om, gm, prec = _models(gpu, name)
+    D = m.cfg.d_model
+    x = np.random.default_rng(B * T).normal(0, 1, (B, T, D)).astype(np.float32)
+    print(f"[layer-rows] {name} B={B} T={T}", flush=True)
+    ref = om.conformer_layer(1, x, oracle.rel_pos_encoding(T, D), valid)
+    dx = gpu.DeviceArray.from_numpy(x, stream)
+    dy = gpu.DeviceArray((B, T, D), np.float32)
+    gm.conformer_layer(1, dx, valid, dy, stream=stream)
+    got, mask = dy.numpy(stream), _valid_mask(B, T, valid)
+    assert rel_l2(got[mask], ref[mask]) < _tol(prec)
+    assert rel_l2(got[mask] - x[mask], ref[mask] - x[mask]) < 3 * _tol(prec)
+    if name == "f16_k5":
+        test_conv_module(gpu, stream, name, B, T, valid)
+
+
 @pytest.mark.parametrize("wt", ["f32", "f16"])
 @pytest.mark.parametrize("B,T,valid", [(3, 1500, [1500, 1499, 3]), (3, 2000, [2000, 64, 1999]), (3, 2100, [2100, 2099, 1]),
                                        (5, 1700, [1700, 1, 33, 1699, 64])])
