@@ -407,11 +407,16 @@ constexpr int SC_TCM = 8;   // chunk frames of the compile-time conv path
 // chain of latencies.  Every global load of a channel (taps, history, chunk,
 // normalisation) is issued before any arithmetic, the outputs stay in registers,
 // all eight waves sum for every frame's normalisation, and the history update is
-// written from registers.  D 512, 2 frames on MI355X, against outputs through LDS
-// and a wave per frame: one stream 7.6 -> 5.7 us, 256 streams 10.0 -> 7.5.
-template <typename T, int K, int TCM, int NC>
+// written from registers.  D 512, 2 frames on MI355X, launched alone, against
+// outputs through LDS and a wave per frame: one stream 5.9 -> 4.0 us, 256 streams
+// 7.2 -> 5.1.  The sums go by DPP: by ds_bpermute they were 4.7 and 5.6, and slower
+// than before from 4 frames on (8 frames 7.1 -> 10.6).
+// WPF: outputs through LDS ([Tc][D]) and a wave per frame, where few channels and
+// many frames leave more to the sums than to the exchange.
+template <typename T, int K, int TCM, int NC, bool WPF>
 __global__ __launch_bounds__(512) void stream_conv_kernel_k(StreamConvParams p) {
     __shared__ float red[2][TCM][8];
+    extern __shared__ float dwo[];               // WPF: [Tc][D]
     constexpr int LP = K - 1;
     const int b = blockIdx.x, D = p.D, Tc = p.Tc;
     const T* glu = (const T*)p.glu + (int64_t)b * Tc * D;
@@ -443,6 +448,7 @@ __global__ __launch_bounds__(512) void stream_conv_kernel_k(StreamConvParams p) 
 #pragma unroll
                 for (int k = 0; k < K; ++k) acc += wk[k] * seq[t + k];
                 y[n][t] = acc + bias;
+                if (WPF) dwo[t * D + c] = y[n][t];
             }
         }
         // history <- the last LP entries of [history ; chunk]
@@ -452,6 +458,22 @@ __global__ __launch_bounds__(512) void stream_conv_kernel_k(StreamConvParams p) 
             for (int t = 0; t <= TCM; ++t)
                 if (t == Tc) hist[(int64_t)j * D + c] = seq[j + t];
         }
+    }
+    if constexpr (WPF) {
+        __syncthreads();
+        for (int t = wid; t < Tc; t += 8) {
+            const float* r = dwo + t * D;
+            float v = 0.f, v2 = 0.f;
+            for (int c = lane; c < D; c += 64) v += r[c];
+            const float mean = wave_sum_full(v) / D;
+            for (int c = lane; c < D; c += 64) v2 += (r[c] - mean) * (r[c] - mean);
+            const float rstd = 1.0f / sqrtf(wave_sum_full(v2) / D + 1e-5f);
+            for (int c = lane; c < D; c += 64) {
+                const float z = (r[c] - mean) * rstd * p.g[c] + p.beta[c];
+                out[(int64_t)t * D + c] = to_act<T>(z / (1.0f + __expf(-z)));
+            }
+        }
+        return;
     }
     if (p.ln) {
         // mean, then the variance about it, each over all waves
@@ -463,7 +485,7 @@ __global__ __launch_bounds__(512) void stream_conv_kernel_k(StreamConvParams p) 
                     float v = 0.f;
 #pragma unroll
                     for (int n = 0; n < NC; ++n) v += pass == 0 ? y[n][t] : y[n][t] * y[n][t];
-                    v = wave_sum(v);
+                    v = wave_sum_full(v);
                     if (lane == 0) red[pass][t][wid] = v;
                 }
             __syncthreads();
@@ -494,11 +516,17 @@ __global__ __launch_bounds__(512) void stream_conv_kernel_k(StreamConvParams p) 
     }
 }
 
+// LayerNorm by a wave per frame from 6 frames at D <= 512 and from 4 at D <= 256 (f16, mean
+// over 1 to 256 streams, us, sums over all waves / a wave per frame: D 512, 5 frames 6.6 /
+// 6.5, 6 7.2 / 6.7, 8 8.5 / 6.9; D 256, 3 frames 4.8 / 4.7, 4 5.4 / 4.9, 8 7.8 / 5.5; D 1024, 8
+// frames: all waves 12.0, against 12.3 with outputs through LDS).
 template <typename T>
 void launch_conv_k(const StreamConvParams& q, int B, hipStream_t s) {
-    if (q.D <= 512) launch(stream_conv_kernel_k<T, 9, SC_TCM, 1>, dim3(B), dim3(512), 0, s, q);
-    else if (q.D <= 1024) launch(stream_conv_kernel_k<T, 9, SC_TCM, 2>, dim3(B), dim3(512), 0, s, q);
-    else launch(stream_conv_kernel_k<T, 9, SC_TCM, 4>, dim3(B), dim3(512), 0, s, q);
+    if (q.D <= 512 && q.ln && q.Tc >= (q.D <= 256 ? 4 : 6))
+        launch(stream_conv_kernel_k<T, 9, SC_TCM, 1, true>, dim3(B), dim3(512), (uint32_t)(q.Tc * q.D * 4), s, q);
+    else if (q.D <= 512) launch(stream_conv_kernel_k<T, 9, SC_TCM, 1, false>, dim3(B), dim3(512), 0, s, q);
+    else if (q.D <= 1024) launch(stream_conv_kernel_k<T, 9, SC_TCM, 2, false>, dim3(B), dim3(512), 0, s, q);
+    else launch(stream_conv_kernel_k<T, 9, SC_TCM, 4, false>, dim3(B), dim3(512), 0, s, q);
 }
 
 }  // namespace

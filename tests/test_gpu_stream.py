@@ -206,6 +206,17 @@ VARIANTS = {
     # rows, the 9-tap conv with two and four channels a thread (not all in range)
     "f32_dk64_d640": (dict(d_model=640, n_heads=10, ff_dim=256), "f32", 0, 1e-4, 25),
     "f32_dk128_batchnorm": (dict(d_model=256, n_heads=2, ff_dim=256, conv_norm_type="batch_norm"), "f32", 0, 1e-4, 25),
+    # the 9-tap conv's frames: all waves a frame (3 at d 256, 8 at d 640), a wave per frame (4 at d 256, 8 at d 512)
+    "f16_tc3_d256": (dict(d_model=256, n_heads=4, ff_dim=256, stream_chunk_size=(9, 24), stream_shift_size=(9, 24),
+                          stream_valid_out_len=3, att_context_right=2), "f16", 1, 1e-2, 33),
+    "q8_0_tc4_d256": (dict(d_model=256, n_heads=4, ff_dim=256, stream_chunk_size=(9, 32), stream_shift_size=(9, 32),
+                           stream_valid_out_len=4, att_context_right=3), "q8_0", 1, 1e-2, 41),
+    "f32_tc8_d512": (dict(d_model=512, n_heads=8, ff_dim=256, stream_chunk_size=(9, 64), stream_shift_size=(9, 64),
+                          stream_valid_out_len=8, att_context_right=7), "f32", 0, 1e-4, 73),
+    "f16_tc6_d512_batchnorm": (dict(d_model=512, n_heads=4, ff_dim=256, stream_chunk_size=(9, 48), conv_norm_type="batch_norm",
+                                    stream_shift_size=(9, 48), stream_valid_out_len=6, att_context_right=5), "f16", 1, 1e-2, 57),
+    "f32_tc8_d640": (dict(d_model=640, n_heads=10, ff_dim=256, stream_chunk_size=(9, 64), stream_shift_size=(9, 64),
+                          stream_valid_out_len=8, att_context_right=7), "f32", 0, 1e-4, 73),
     "f16_dk128_d1152": (dict(d_model=1152, n_heads=9, ff_dim=256), "f16", 1, 1e-2, 25),
 }
 
