@@ -144,12 +144,14 @@ __device__ __forceinline__ void stream_attn_finish(const StreamAttnParams& p, in
 // issued together), a wave a softmax row, and a thread 16 bytes of one
 // query's output channels.  Keeping only the values in LDS lets the whole
 // grid of a step (streams x heads) be resident at once.  For the head widths that
-// stream_attn_rows_kernel is not made for.
-template <typename T>
+// stream_attn_rows_kernel is not made for, and the steps where it is slower
+// (launch_stream_attn).  DK > 0: the head width at compile time (dot products fully
+// unrolled); DK = 0 reads it from p.dk.
+template <typename T, int DK>
 __global__ __launch_bounds__(256) void stream_attn_kernel(StreamAttnParams p) {
     extern __shared__ float sm[];
     constexpr int VE = 16 / sizeof(T);           // elements per 16-byte vector
-    const int b = blockIdx.x, h = blockIdx.y, dk = p.dk, D = p.D, Tc = p.Tc, CL = p.CL;
+    const int b = blockIdx.x, h = blockIdx.y, dk = DK > 0 ? DK : p.dk, D = p.D, Tc = p.Tc, CL = p.CL;
     const int Tk = CL + Tc, ld = dk + VE;
     float* qu = sm;                              // [Tc][dk]
     float* qv = qu + Tc * dk;                    // [Tc][dk]
@@ -225,10 +227,11 @@ __global__ __launch_bounds__(256) void stream_attn_kernel(StreamAttnParams p) {
 // (the rings' 37 MB take 7.7 at the rate of a large copy; 128 VGPRs leave four of
 // eight workgroups a CU resident, and bounds that fit more spill); one stream
 // 8.3 -> 7.2.
+constexpr int SA_NB = 3;   // rows of each kind a thread has in flight
 template <typename T, int DK>
 __global__ __launch_bounds__(256) void stream_attn_rows_kernel(StreamAttnParams p) {
     extern __shared__ float sm[];
-    constexpr int VE = 16 / sizeof(T), VPR = DK / VE, RP = 256 / VPR, NB = 3, LD = DK + VE;
+    constexpr int VE = 16 / sizeof(T), VPR = DK / VE, RP = 256 / VPR, NB = SA_NB, LD = DK + VE;
     const int b = blockIdx.x, h = blockIdx.y, D = p.D, Tc = p.Tc, CL = p.CL, Tk = CL + Tc;
     float* qu = sm;                              // [Tc][DK]
     float* qv = qu + Tc * DK;                    // [Tc][DK]
@@ -322,6 +325,26 @@ __global__ __launch_bounds__(256) void stream_attn_rows_kernel(StreamAttnParams 
         }
     }
     stream_attn_finish<T>(p, DK, sc, vs);
+}
+
+// The step on the faster of the two kernels.  Past two queries the rows kernel
+// loads positional rows in every pair of queries of every batch of rows, also of a
+// last batch that is nearly empty, and with at most one workgroup per CU nothing
+// covers them; 32 lanes a row (f32, heads of 128) leave small batches.  Sweep on
+// MI355X over 1 to 32 frames, 70 cached, 1 to 256 streams, 4 and 8 heads (us, rows
+// kernel / score a thread, 8 heads; f16, 64 wide: 1 stream, 24 frames, one batch, 25.4 /
+// 28.6, 28 frames, two, 39.2 / 33.8, 256 streams 137 / 224; 128 wide: 1 stream, 24 frames
+// 46.5 / 47.7, 28 64.9 / 56.7, 64 streams 77 / 105; f32, 128 wide: 1 stream, 8 frames 26.8 /
+// 25.9, 28 103 / 89, 256 streams, 8 frames 122 / 165, 28 863 / 777).
+template <typename T, int DK> void launch_stream_attn(const StreamAttnParams& a, dim3 grid, uint32_t shm, hipStream_t s) {
+    constexpr int VPR = DK * (int)sizeof(T) / 16, ROWS = SA_NB * (256 / VPR);   // rows of a batch
+    const int Tk = a.CL + a.Tc;
+    const bool many = (int64_t)grid.x * grid.y > device_cu_count();
+    bool rows = a.Tc <= 2;
+    if (!rows && VPR >= 32) rows = a.Tc <= 7 || (many && a.Tc < 24);
+    else if (!rows) rows = many || 10 * ROWS * cdiv(Tk, ROWS) <= 14 * Tk;   // batches not mostly empty
+    if (rows) launch(stream_attn_rows_kernel<T, DK>, grid, dim3(256), shm, s, a);
+    else launch(stream_attn_kernel<T, DK>, grid, dim3(256), shm, s, a);
 }
 
 struct StreamConvParams {
@@ -547,7 +570,9 @@ std::unique_ptr<StreamState> Model::stream_create(int n_streams, int max_window,
             "streaming encoder: d_model above 2048, or head width above 256 or not a multiple of 8");
     // LDS beyond the default 64 KiB (attention: stream_attn_lds_bytes, conv:
     // SC_FRAMES x D floats)
-    for (const void* fn : {(const void*)stream_attn_kernel<f16>, (const void*)stream_attn_kernel<float>,
+    for (const void* fn : {(const void*)stream_attn_kernel<f16, 0>, (const void*)stream_attn_kernel<float, 0>,
+                           (const void*)stream_attn_kernel<f16, 64>, (const void*)stream_attn_kernel<float, 64>,
+                           (const void*)stream_attn_kernel<f16, 128>, (const void*)stream_attn_kernel<float, 128>,
                            (const void*)stream_attn_rows_kernel<f16, 64>, (const void*)stream_attn_rows_kernel<float, 64>,
                            (const void*)stream_attn_rows_kernel<f16, 128>, (const void*)stream_attn_rows_kernel<float, 128>,
                            (const void*)stream_conv_kernel<f16>, (const void*)stream_conv_kernel<float>})
@@ -693,13 +718,13 @@ int Model::stream_step(StreamState& st, const float* mel, int n, bool is_last, f
             mark(KF_ATTENTION, true);
             const dim3 grid(B, H);
             if (prec_ == PREC_F16) {
-                if (dk == 64) launch(stream_attn_rows_kernel<f16, 64>, grid, dim3(256), shm, s, a);
-                else if (dk == 128) launch(stream_attn_rows_kernel<f16, 128>, grid, dim3(256), shm, s, a);
-                else launch(stream_attn_kernel<f16>, grid, dim3(256), shm, s, a);
+                if (dk == 64) launch_stream_attn<f16, 64>(a, grid, shm, s);
+                else if (dk == 128) launch_stream_attn<f16, 128>(a, grid, shm, s);
+                else launch(stream_attn_kernel<f16, 0>, grid, dim3(256), shm, s, a);
             } else {
-                if (dk == 64) launch(stream_attn_rows_kernel<float, 64>, grid, dim3(256), shm, s, a);
-                else if (dk == 128) launch(stream_attn_rows_kernel<float, 128>, grid, dim3(256), shm, s, a);
-                else launch(stream_attn_kernel<float>, grid, dim3(256), shm, s, a);
+                if (dk == 64) launch_stream_attn<float, 64>(a, grid, shm, s);
+                else if (dk == 128) launch_stream_attn<float, 128>(a, grid, shm, s);
+                else launch(stream_attn_kernel<float, 0>, grid, dim3(256), shm, s, a);
             }
             PKX_LAUNCH_CHECK();
             mark(KF_ATTENTION, false);

@@ -217,6 +217,15 @@ VARIANTS = {
                                     stream_shift_size=(9, 48), stream_valid_out_len=6, att_context_right=5), "f16", 1, 1e-2, 57),
     "f32_tc8_d640": (dict(d_model=640, n_heads=10, ff_dim=256, stream_chunk_size=(9, 64), stream_shift_size=(9, 64),
                           stream_valid_out_len=8, att_context_right=7), "f32", 0, 1e-4, 73),
+    # steps on the other side of the attention kernels' rule: a second batch of rows nearly empty, f32 heads of 128
+    "f16_tc28": (dict(d_model=256, n_heads=4, ff_dim=256, stream_chunk_size=(9, 224), stream_shift_size=(9, 224),
+                      stream_valid_out_len=28, att_context_right=27), "f16", 1, 1e-2, 233),
+    "f16_dk128_tc28": (dict(d_model=256, n_heads=2, ff_dim=256, stream_chunk_size=(9, 224), stream_shift_size=(9, 224),
+                            stream_valid_out_len=28, att_context_right=27), "f16", 1, 1e-2, 233),
+    "f32_dk64_tc28": (dict(d_model=128, n_heads=2, ff_dim=256, stream_chunk_size=(9, 224), stream_shift_size=(9, 224),
+                           stream_valid_out_len=28, att_context_right=27), "f32", 0, 1e-4, 233),
+    "f32_dk128_tc10": (dict(d_model=256, n_heads=2, ff_dim=256, stream_chunk_size=(9, 80), stream_shift_size=(9, 80),
+                            stream_valid_out_len=10, att_context_right=9), "f32", 0, 1e-4, 89),
     "f16_dk128_d1152": (dict(d_model=1152, n_heads=9, ff_dim=256), "f16", 1, 1e-2, 25),
 }
 
@@ -228,7 +237,7 @@ def test_streaming_variants_match_oracle(gpu, stream, name):
     m = pm.synthesize(cfg, qt, heads=False, std=0.05, bn_random=True)
     om = oracle.OracleModel(m)
     gm = gpu.Model.from_tensors(m, precision=prec)
-    S, T = 2, 200
+    S, T = 2, 200 if max_window < 200 else 3 * max_window
     rng = np.random.default_rng(21)
     mels = rng.normal(0, 1, (S, cfg.n_mels, T)).astype(np.float32)
     st = gpu.Streaming(gm, n_streams=S, max_window=max_window, stream=stream)
@@ -253,5 +262,7 @@ def test_streaming_variants_match_oracle(gpu, stream, name):
     print(f"[stream]   worst chunk rel_l2 {worst:.2e}", flush=True)
     if "tc9" in name:
         assert max(tcs) > 8
+    if "tc28" in name:
+        assert max(tcs) == 28
     st.close()
     gm.close()
