@@ -607,7 +607,7 @@ __global__ __launch_bounds__(512, 1) void relpos_attn_long_kernel(AttnParams a) 
         for (int g = 0; g < NGR; ++g) {
             if (g + 2 < NGR) fetch(g + 2);
             // G's first half leaves while K's products run
-            if (g == NKC + 1 || (NGR == 2 && g == 1)) {
+            if (g == NKC + 1) {   // NKC >= 2
 #pragma unroll
                 for (int gt = 0; gt < 3; ++gt) *(float4v*)(garea + 16 * gt) = gb[gt];
             }
@@ -947,6 +947,12 @@ __global__ __launch_bounds__(64) void relpos_attn_f32_kernel(AttnParams a, int d
     }
 }
 
+void attention_f32_ready() {
+    for (const void* fn : {(const void*)relpos_attn_f32_mfma_kernel<32>, (const void*)relpos_attn_f32_mfma_kernel<64>,
+                           (const void*)relpos_attn_f32_mfma_kernel<128>})
+        PKX_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+}
+
 void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s) {
     require(a.T > 0 && a.B > 0 && a.H > 0, "attention: empty shape");
     if (prec == PREC_F16) {
@@ -1006,8 +1012,6 @@ void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s)
         const size_t sm16 = attn_f32_mfma_lds(a.T);
         auto go = [&](auto DKc) {
             auto* fn = relpos_attn_f32_mfma_kernel<decltype(DKc)::value>;
-            if (sm16 > 64 * 1024)
-                PKX_HIP(hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
             launch(fn, dim3(cdiv(a.T, 16), a.H, a.B), dim3(256), (uint32_t)sm16, s, a);
         };
         if (rows16 && sm16 <= 160 * 1024 && a.dk == 128) go(std::integral_constant<int, 128>{});

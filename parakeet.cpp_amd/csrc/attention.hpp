@@ -22,4 +22,8 @@ struct AttnParams {
 
 void launch_relpos_attention(Precision prec, const AttnParams& a, hipStream_t s);
 
+// On the current device, once before the f32 path runs there: lets its matrix
+// kernel take more than the default 64 KB of LDS.
+void attention_f32_ready();
+
 }  // namespace pkx

@@ -688,6 +688,7 @@ void Model::finalize() {
         PKX_HIP(hipDeviceSynchronize());
     }
     host_.clear();
+    if (prec_ == PREC_F32) attention_f32_ready();
     // split-K workspace (residual products of few rows): created here, once, so
     // that no forward or streaming step allocates or synchronises for it
     grow(ws_->skpart, (size_t)SK_FLOATS * 4);
