@@ -263,6 +263,6 @@ def test_streaming_variants_match_oracle(gpu, stream, name):
     if "tc9" in name:
         assert max(tcs) > 8
     if "tc28" in name:
-        assert max(tcs) == 28
+        assert max(tcs) == 30   # of which a step drops 2
     st.close()
     gm.close()
