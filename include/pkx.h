@@ -234,8 +234,7 @@ int pkx_linear(int precision, int ggml_type, int N, int K, const void* host_w, s
 /* y += alpha * (x . W^T + bias): the residual products of the encoder
  * (ggml_add(r, ggml_scale(ggml_mul_mat(W, x), 0.5)), src/conformer.cpp:326-330,
  * with alpha 0.5; alpha 1 for linear_out / pointwise_conv2) on the kernels the
- * encoder runs them with, including the split-K path for products of at most
- * 512 rows and K >= 1024.  y_dev [M][N] f32, read and written. */
+ * encoder runs them with.  y_dev [M][N] f32, read and written. */
 int pkx_linear_residual(int precision, int ggml_type, int N, int K, const void* host_w, size_t nbytes,
                         const float* bias_dev, const float* x_dev, int64_t M, float alpha, float* y_dev,
                         void* stream);

@@ -1110,15 +1110,8 @@ struct FoldStats {
 // by side along N, each 64 TM rows x 16 TN columns, so that no two waves
 // dequantise the same weight rows; 2 = the 2 x 2 layout with the slab's LDS
 // reads issued up front (as layout 1 does).
-// WL = 3: layout 0 with the K range cut over p.ksplit workgroups per tile
-// (split-K across workgroups, for grids far smaller than the chip).  Each
-// workgroup writes its partial tile to p.sk_part and counts itself in
-// p.sk_cnt[tile]; the last one to arrive sums the partials in split order (the
-// same order whichever arrives last, so results are deterministic), resets the
-// counter and runs the epilogue.
 template <int TM, int TN, int WT, int EPI, int NS = DMA_NS, int KG = 1, int WL = 0>
 __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void gemm_dma_kernel(GemmParams p) {
-    constexpr bool SPLIT = WL == 3;
     typedef DmaCfg<TM, TN, WT> C;
     static_assert(WL != 1 || (TN % 2 == 0 && EPI != EPI_GLU && EPI != EPI_GLU_DW && EPI != EPI_RELU_TR &&
                               EPI != EPI_RELU2_F32),
@@ -1141,18 +1134,8 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void gemm_dma_kernel(Gem
     constexpr int DWH = EPI == EPI_GLU_DW ? (GLU_DW_K - 1) / 2 : 0;
     constexpr int SM = C::BM - 2 * DWH;
     const int nbm = cdiv_dev(p.M, SM), nbn = cdiv_dev(p.N, C::BN);
-    int bm, bn, tile = 0, split = 0;
-    if constexpr (SPLIT) {
-        // the splits of one tile are consecutive positions: usually on one XCD,
-        // but they straddle two whenever an XCD's range of positions is not a
-        // multiple of ksplit, so the handoff below is made coherent across XCDs
-        const int k = xcd_tile(blockIdx.x, nbm * nbn * p.ksplit);
-        tile = k / p.ksplit;
-        split = k - tile * p.ksplit;
-        xcd_rect(tile, nbm, nbn, p.xcd_gm, bm, bn);
-    } else {
-        xcd_tile_2d(blockIdx.x, nbm, nbn, p.xcd_gm, bm, bn);
-    }
+    int bm, bn;
+    xcd_tile_2d(blockIdx.x, nbm, nbn, p.xcd_gm, bm, bn);
     const int m0 = bm * SM - DWH, n0 = bn * C::BN;
 
     float16v acc[WTM][WTN];
@@ -1177,7 +1160,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void gemm_dma_kernel(Gem
     // tile: group g sums and runs the epilogue of row block g (the other
     // group's partial of it comes through LDS), so both groups' waves work in
     // the reduction and the epilogue instead of group 0's alone.
-    constexpr bool KHALF = KG == 2 && WTM == 2 && !SPLIT && whole;
+    constexpr bool KHALF = KG == 2 && WTM == 2 && whole;
     constexpr int ER = KHALF ? 32 : 32 * WTM;   // rows of this wave's epilogue
     const int erow = wm * WTM * 32 + (KHALF ? kg * 32 : 0);   // its first row within the tile
     const bool epi_wave = KHALF || kg == 0;
@@ -1194,7 +1177,7 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void gemm_dma_kernel(Gem
     if constexpr (EPI == EPI_GLU_DW) dwpre.load(p, m0, n0, tid);
 
     // slabs of this group, its first K
-    const int nk = SPLIT ? p.K / 64 / KG / p.ksplit : p.K / 64 / KG, kb = (split * KG + kg) * nk * 64;
+    const int nk = p.K / 64 / KG, kb = kg * nk * 64;
     DmaSrc<TM, TN, WT> src;
     src.init(p, m0, n0, wid, lane);
     src.issue(smem, kb);
@@ -1270,73 +1253,6 @@ __global__ __launch_bounds__(256 * KG, KG == 1 ? 2 : 1) void gemm_dma_kernel(Gem
                 for (int j = 0; j < WTN; ++j)
 #pragma unroll
                     for (int r = 0; r < 16; ++r) acc[i][j][r] += red[((i * WTN + j) * 16 + r) * 64];
-        }
-    }
-    if constexpr (SPLIT) {
-        static_assert(!FOLD && EPI != EPI_GLU_DW, "split-K: no folded LayerNorm");
-        // Partial tiles [tile][split][wave][register][lane].  Why the relaxed
-        // accesses below suffice on gfx950 (the C++ model alone would ask for
-        // release / acquire): every access to the partials and the counter is
-        // an agent-scope atomic, which gfx950 performs at the device's point of
-        // coherence (the store writes through the XCD's L2, the load does not
-        // take a possibly stale L2 line), whichever XCD issues it.  A writer
-        // (1) stores its partial, (2) waits with s_waitcnt vmcnt(0), which
-        // returns only once those stores are acknowledged at that scope, and
-        // only then (3) issues its counter increment; the last arriver's
-        // increment is ordered after every writer's (one location, one
-        // modification order), and its partial loads are issued only after the
-        // increment has returned.  So each partial it loads was complete at the
-        // coherence point before it was read.  An agent-scope release / acquire
-        // fence would add a write-back and an invalidation of the whole L2 of
-        // the XCD, evicting the weights every other workgroup is streaming
-        // (57 us per launch against 7.7 - 14 us, measured); that is the only
-        // thing it would add here, since no plain (cacheable) access carries
-        // data between the workgroups.
-        constexpr int R = WTM * WTN * 16;
-        const int S = p.ksplit;
-        float* part = p.sk_part + (int64_t)tile * S * (4 * R * 64) + wid * R * 64 + lane;
-        if (kg == 0) {
-#pragma unroll
-            for (int i = 0; i < WTM; ++i)
-#pragma unroll
-                for (int j = 0; j < WTN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r)
-                        __hip_atomic_store(part + (int64_t)split * (4 * R * 64) + ((i * WTN + j) * 16 + r) * 64,
-                                           acc[i][j][r], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            wait_vmcnt<0>();   // the partial has reached the device before the count
-        }
-        __shared__ int sk_last;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const int seen = __hip_atomic_fetch_add(p.sk_cnt + tile, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            sk_last = seen == S - 1;
-            // every split of this tile has counted: ready for the next launch
-            if (seen == S - 1) __hip_atomic_store(p.sk_cnt + tile, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        if (!sk_last) return;
-        if (kg == 0) {
-            // the sum in split order, whichever split arrived last
-            float16v own[WTM][WTN];
-#pragma unroll
-            for (int i = 0; i < WTM; ++i)
-#pragma unroll
-                for (int j = 0; j < WTN; ++j) own[i][j] = acc[i][j];
-            for (int t = 0; t < S; ++t) {
-#pragma unroll
-                for (int i = 0; i < WTM; ++i)
-#pragma unroll
-                    for (int j = 0; j < WTN; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            const float v = t == split ? own[i][j][r]
-                                                       : __hip_atomic_load(part + (int64_t)t * (4 * R * 64) +
-                                                                               ((i * WTN + j) * 16 + r) * 64,
-                                                                           __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                            acc[i][j][r] = t == 0 ? v : acc[i][j][r] + v;
-                        }
-            }
         }
     }
     // folded LayerNorm: the tile's row statistics at the top of the LDS block
@@ -2504,29 +2420,6 @@ static void dma_22q(int epi, const GemmParams& p, hipStream_t s) {
     default: dma_epi<2, 2, WT>(epi, p, s); break;
     }
 }
-// Split-K across workgroups for the residual products of few rows and K >= 1024
-// that the K-split tiles do not take (N no multiple of 32, unaligned operands): 64 x 64 tiles in two K groups, the K range cut over S workgroups
-// per tile (S a power of two up to 8, each K group keeping at least one 64-deep
-// slab) until the grid holds about one workgroup per CU.  On MI355X at M = 512,
-// N = 512, K = 2048: 64 tiles x 4 splits, 1.4 us faster per launch; at K = 512
-// (linear_out, pw2) and with two workgroups per CU it was slower.
-template <int WT>
-static bool dma_splitk(int epi, const GemmParams& p, hipStream_t s) {
-    if (!p.sk_part || !p.sk_cnt || p.M > 512 || p.K < 1024 || (epi != EPI_RESID && epi != EPI_RESID_LN))
-        return false;
-    const int tiles = cdiv(p.M, 64) * cdiv(p.N, 64);
-    const int cus = device_cu_count();
-    int S = 1;
-    while (S < 8 && 2 * S * tiles <= cus && p.K % (2 * S * 128) == 0) S *= 2;
-    if (S == 1 || (int64_t)tiles * S * 64 * 64 > p.sk_part_floats || tiles > p.sk_cnt_n) return false;
-    GemmParams q = p;
-    q.ksplit = S;
-    q.xcd_gm = choose_xcd_gm(p, WT, 64, 64);
-    if (epi == EPI_RESID) launch((gemm_dma_kernel<1, 1, WT, EPI_RESID, DMA_NS, 2, 3>), dim3(tiles * S), dim3(512), 0, s, q);
-    else launch((gemm_dma_kernel<1, 1, WT, EPI_RESID_LN, DMA_NS, 2, 3>), dim3(tiles * S), dim3(512), 0, s, q);
-    PKX_LAUNCH_CHECK();
-    return true;
-}
 // 128 x 64 tiles with two K groups (eight waves): products of K >= 1024 whose
 // grid is about one tile per CU and that the register-B kernels do not take
 // (pw2 with f16 weights at K = 1024; the split took 0.3 - 0.9 us off a
@@ -2747,9 +2640,6 @@ void launch_gemm(Precision prec, int wtype, int epi, const GemmParams& p, hipStr
         if (wtype == GT_Q4_K && dma_rb<GT_Q4_K>(epi, p, s)) return;
         if (wtype == GT_Q8_0 && dma_rb_resid<GT_Q8_0>(epi, p, s)) return;
         if (wtype == GT_Q4_K && dma_rb_resid<GT_Q4_K>(epi, p, s)) return;
-        if (wtype == GT_Q8_0 && dma_splitk<GT_Q8_0>(epi, p, s)) return;
-        if (wtype == GT_Q4_K && dma_splitk<GT_Q4_K>(epi, p, s)) return;
-        if (wtype == GT_F16 && dma_splitk<GT_F16>(epi, p, s)) return;
         if (wtype == GT_Q8_0 && dma_kg2<GT_Q8_0>(epi, p, s)) return;
         if (wtype == GT_Q4_K && dma_kg2<GT_Q4_K>(epi, p, s)) return;
         if (wtype == GT_F16 && dma_kg2<GT_F16>(epi, p, s)) return;

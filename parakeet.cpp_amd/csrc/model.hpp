@@ -239,9 +239,6 @@ private:
     void gemm_resid_ln(const DevWeight& w, const void* A, int64_t M, const float* bias, float* x, float alpha,
                        const float* g, void* h, hipStream_t s, int fam, const float* res_rows = nullptr,
                        const float* res_g = nullptr, const float* res_b = nullptr);
-    // split-K workspace for residual products of few rows (M <= 512), made on
-    // first use; launch_gemm decides whether to split
-    void splitk_ws(GemmParams& p, hipStream_t s);
     // product of a LayerNorm folded in (A = x * gamma from gemm_resid_ln)
     GemmParams fold_params(const DevWeight& w, const void* A, int64_t M, const float* c1, const float* c2,
                            void* Y, int64_t ldy);
@@ -301,8 +298,7 @@ DevWeight weight_rows_view(const DevWeight& w, int row0, int nrows);
 
 // y[M][N] = x[M][K] . W^T (+ bias) for one raw weight, f32 in/out; the weight
 // is uploaded for this call and freed after the stream drains.  residual:
-// y += alpha (x . W^T + bias) instead (the encoder's residual product, with
-// its split-K path for few rows).
+// y += alpha (x . W^T + bias) instead (the encoder's residual product).
 void linear_raw(Precision prec, const HostTensor& t, int N, int K, const float* bias, const float* x,
                 int64_t M, float* y, hipStream_t s, bool residual = false, float alpha = 1.0f);
 

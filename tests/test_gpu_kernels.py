@@ -157,17 +157,15 @@ def _residual_calls(gpu, stream, gtype, K, shapes, rng, tag):
 
 
 @pytest.mark.parametrize("gtype", [pm.GGML_Q8_0, pm.GGML_F16])
-def test_residual_split_k_fresh_inputs(gpu, stream, gtype):
-    """The split-K residual product (M <= 512 rows, K >= 1024: S workgroups per
-    tile hand partial tiles to the last arriver, which sums them in split order)
-    on fresh random inputs at every call, the calls of different sizes (some
-    with a tile's splits on two XCDs), so a stale or missing partial cannot
-    repeat the previous result."""
-    # (M, N): 128 64x64 tiles x 2 splits and 64 x 4 (32 positions per XCD, a
-    # tile's splits on one XCD), then 10 tiles x 8 splits and 21 x 4, whose
-    # per-XCD ranges (10, 10-11 positions) cut tiles' splits over two XCDs
-    _residual_calls(gpu, stream, gtype, 2048, ((512, 1024), (200, 1024), (128, 320), (192, 448), (512, 1024)),
-                    _rng(2048), "split-k")
+def test_residual_few_rows_fresh_inputs(gpu, stream, gtype):
+    """The residual product of few rows (K split over the waves of a workgroup,
+    the partial tiles summed in a fixed order) on fresh random inputs at every
+    call, the calls of different sizes, so a stale or missing partial cannot
+    repeat the previous result; and with N no multiple of 32, which the K-split
+    tiles do not take (64 x 64 tiles with two K groups)."""
+    _residual_calls(gpu, stream, gtype, 2048, ((512, 1024), (200, 1024), (128, 320), (192, 448), (512, 1024),
+                                               (128, 312), (512, 488), (125, 1000)),
+                    _rng(2048), "few-rows")
 
 
 @pytest.mark.parametrize("gtype", [pm.GGML_Q8_0, pm.GGML_F16])

@@ -14,8 +14,8 @@ oracle, through the C ABI.
   1e-2, then the TDT joint (640 hidden, 1025 tokens + 5 durations) argmax.
 * 1.1B-shape q8_0 encoder, 42 blocks, the configuration's 8 clips of 30 s
   (T' 375, one of them ragged), every layer within 1e-2.
-* 0.6B shape, 3 blocks, at few rows (B 3 ragged and B 1): the split-K
-  residual products, every layer within 1e-2 and bit-identical on a repeat.
+* 0.6B shape, 3 blocks, at few rows (B 3 ragged and B 1): the residual
+  products on the few-row kernel, every layer within 1e-2 and bit-identical on a repeat.
 Relative L2 is over each item's valid frames.
 """
 import time
@@ -210,12 +210,12 @@ def test_06b_full_depth_f16_ragged_tdt(gpu, stream):
 
 
 # ---------------------------------------------------------------------------
-# Few rows (M = B*T' <= 512): the residual products of K >= 1024 (FFN linear2,
-# attention out, pw2) split K over 2 (B 3, M 375) or 8 (B 1, M 125) workgroups
-# per tile, partials summed in a fixed order
+# Few rows (B 3, M = B*T' = 375 and B 1, M 125): the residual products on the
+# few-row kernel, K split over the waves of a workgroup, partials summed in a
+# fixed order
 # ---------------------------------------------------------------------------
 @pytest.mark.parametrize("wtype,lens", [("q8_0", [1000, 737, 1000]), ("f16", [1000])])
-def test_06b_few_rows_split_k(gpu, stream, wtype, lens):
+def test_06b_few_rows(gpu, stream, wtype, lens):
     m = pm.synthesize(_cfg06(3), wtype, bn_random=True, heads=False)
     om = oracle.OracleModel(m)
     gm = gpu.Model.from_tensors(m, gpu.PREC_F16)
@@ -223,7 +223,7 @@ def test_06b_few_rows_split_k(gpu, stream, wtype, lens):
     mel = rng.normal(0, 1, (len(lens), 128, 1000)).astype(np.float32)
     for b, v in enumerate(lens):
         mel[b, :, v:] = 0.0
-    label = f"split-K {wtype} B={len(lens)}"
+    label = f"few rows {wtype} B={len(lens)}"
     print(f"[{label}] lens={lens}", flush=True)
     got, _, _ = _run_encoder(gpu, stream, gm, om, mel, lens, label, 1e-2)
     # deterministic: the same partials in the same order on a second call
