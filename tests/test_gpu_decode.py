@@ -5,6 +5,7 @@ frames and spans per item (the argmax decisions), confidence within 1e-5.
 The joint's output weights are scaled up so that the decisions have margins
 far above f32 rounding (the device sums the products in another order)."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -196,3 +197,67 @@ def test_greedy_decode_leaves_no_earlier_tokens(gpu, stream):
         most = cnt if most is None else most
     assert (cnt < most).all()
     d_enc.free()
+
+
+def _check_items(got, want, tol=1e-5):
+    for b, (g, w) in enumerate(zip(got, want)):
+        for i in (0, 1, 3):
+            assert np.array_equal(g[i], w[i]), (b, i, g[i][:20], w[i][:20])
+        assert np.max(np.abs(g[2] - w[2]), initial=0.0) <= tol
+
+
+def test_greedy_decode_two_threads_one_model(gpu):
+    """Two host threads decode different batches on one model, each on a stream
+    of its own: the model's working memory goes to one call at a time, the
+    other uses its own."""
+    durations = (0, 1, 2, 3, 4)
+    cfg, m = _model(durations, seed=3)
+    gm, tr = gpu.Model.from_tensors(m), oracle.Transducer(m)
+    rng = np.random.default_rng(33)
+    jobs = []
+    for B, T in ((3, 50), (18, 20)):
+        enc = rng.standard_normal((B, T, cfg.d_model)).astype(np.float32)
+        T_valid = [T] + [int(t) for t in rng.integers(0, T + 1, B - 1)]
+        want = [tr.greedy(enc[b, :T_valid[b]], durations=durations, max_symbols=10) for b in range(B)]
+        s = gpu.Stream()
+        jobs.append((gpu.DeviceArray.from_numpy(enc, s), T_valid, want, s))
+        s.sync()
+    go, failed = threading.Barrier(2), []
+
+    def work(job):
+        d_enc, T_valid, want, s = job
+        try:
+            for call in range(8):
+                go.wait(30)
+                _check_items(gm.transducer_greedy(d_enc, T_valid, durations=durations, stream=s), want)
+        except BaseException as e:   # noqa: BLE001 - reported by the test below
+            failed.append(e)
+            go.abort()
+
+    print(f"[decode] two threads, T={[j[1] for j in jobs]}", flush=True)
+    threads = [threading.Thread(target=work, args=(j,)) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not failed, failed
+    for j in jobs:
+        j[0].free()
+
+
+def test_greedy_decode_past_the_kept_workspace(gpu, stream):
+    """A call whose encoder projections alone exceed the 64 MB that stay with the
+    model, then a small one."""
+    durations = (0, 1, 2, 3, 4)
+    cfg, m = _model(durations, seed=4)
+    gm, tr = gpu.Model.from_tensors(m), oracle.Transducer(m)
+    rng = np.random.default_rng(44)
+    for B, T_max in ((16, 8300), (2, 30), (16, 8300)):
+        T_valid = [int(t) for t in rng.integers(1, 31, B)]
+        enc = np.zeros((B, T_max, cfg.d_model), np.float32)
+        enc[:, :30] = rng.standard_normal((B, 30, cfg.d_model))
+        print(f"[decode] B={B} T_max={T_max} T={T_valid}", flush=True)
+        d_enc = gpu.DeviceArray.from_numpy(enc, stream)
+        got = gm.transducer_greedy(d_enc, T_valid, durations=durations, cap=400, stream=stream)
+        _check_items(got, [tr.greedy(enc[b, :T_valid[b]], durations=durations, max_symbols=10) for b in range(B)])
+        d_enc.free()
