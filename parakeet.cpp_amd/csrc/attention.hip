@@ -458,11 +458,13 @@ __global__ __launch_bounds__(64 * NQW * NG, 1) void relpos_attn_ks_kernel(AttnPa
 // eight waves of 16 queries (two per SIMD), keys in steps of 64, the products
 // formed as in relpos_attn_ks_kernel.
 //
-// What bounds it is LDS bandwidth: a wave reads its step's K, band and V (52 KB
-// at DK = 128) and passes G through it, about 4.9 k cycles a step for the eight
-// waves with the bank conflicts, of the 5.6 k a step takes (MFMA 1.7 k per
-// SIMD).  The loads run a step ahead: K and V have two buffers each, and the
-// positional band is a ring of 256 rows of which a step uses 192 and the next
+// No unit is saturated.  Of the 5.6 k cycles a step takes (4 x 3750 frames,
+// counters) the LDS works 55% (a wave reads its step's K, band and V, 52 KB at
+// DK = 128, and passes G through it; 14% are bank conflicts), the matrix pipe 30%
+// (1.7 k per SIMD), and vector instructions, MFMA among them, issue in 50%; the two
+// waves of a SIMD cover each other only in part and spend 15% of their time
+// waiting on LDS.  The loads run a step ahead: K and V have two buffers each, and
+// the positional band is a ring of 256 rows of which a step uses 192 and the next
 // needs only 64 new ones (a third of the band's traffic), so one step's DMA is
 // 48 KB instead of 80 and has a whole step to land, behind one barrier.  Tiles
 // without a masked key skip the mask arithmetic, and the output is rescaled

@@ -3,11 +3,11 @@
 // subsampling of every stream's mel window, drops the pre-encode overlap,
 // then for each conformer layer the products of the offline path (M = B x Tc
 // rows) around two step kernels:
-//   * stream_attn_rows_kernel: relative-position attention of the chunk's Tc
+//   * launch_stream_attn's kernels: relative-position attention of the chunk's Tc
 //     queries over [cache ; chunk] keys with the streaming mask (empty cache
 //     slots, chunked-limited window; streaming_encoder.cpp:146-245), then the
 //     chunk's keys and values enter the per-layer ring;
-//   * stream_conv_kernel: causal depthwise conv over [GLU history ; chunk]
+//   * the stream_conv kernels: causal depthwise conv over [GLU history ; chunk]
 //     + bias, LayerNorm (or folded BatchNorm) over channels, SiLU
 //     (streaming_encoder.cpp:268-326), then the history advances.
 #include <cmath>
