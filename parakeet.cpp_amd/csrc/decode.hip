@@ -61,6 +61,7 @@ struct MmArgs {
     const float* W;   // [row tiles][chunks][64][4]
     const float* bias;
     int chunks, B;
+    int block0;       // first 16-item block of the launch
     int n_out;        // MM_LSTM: hidden units H (tile row 4 u + g: gate g of unit 4 tile + u); else output rows
     float* y;         // MM_JOINT: dec_at order over y_chunks; MM_PLAIN: [B][n_out]
     int y_chunks;
@@ -86,10 +87,10 @@ __global__ __launch_bounds__(512) void dec_mm_kernel(MmArgs a, DecState st) {
     __shared__ float4v red[8][64];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
-    const int tile = blockIdx.x, b = 16 * blockIdx.y + lr;
+    const int tile = blockIdx.x, ib = a.block0 + blockIdx.y, b = 16 * ib + lr;
     const int c0 = a.chunks * w / 8, nc = a.chunks * (w + 1) / 8 - c0;   // <= MAXC
     const float4v* W = (const float4v*)a.W + ((int64_t)tile * a.chunks + c0) * 64 + lane;
-    const float4v* x = (const float4v*)a.x + ((int64_t)blockIdx.y * a.chunks + c0) * 64 + lane;
+    const float4v* x = (const float4v*)a.x + ((int64_t)ib * a.chunks + c0) * 64 + lane;
     const float4v zero = {0.f, 0.f, 0.f, 0.f};
     float4v wv[MAXC], xv[MAXC];
 #pragma unroll
@@ -364,14 +365,17 @@ struct Carve {
     }
 };
 
+// One workgroup per row tile and 16-item block, a launch per 65535 blocks (the grid's second dimension).
 template <int MODE>
-void launch_mm(const MmArgs& a, const DecState& st, int tiles, hipStream_t s) {
-    const dim3 grid(tiles, cdiv(a.B, 16));
-    const int per = cdiv(a.chunks, 8);   // chunks of a wave
-    if (per <= 5) launch(dec_mm_kernel<MODE, 5>, grid, dim3(512), 0, s, a, st);
-    else if (per <= 10) launch(dec_mm_kernel<MODE, 10>, grid, dim3(512), 0, s, a, st);
-    else launch(dec_mm_kernel<MODE, 16>, grid, dim3(512), 0, s, a, st);
-    PKX_LAUNCH_CHECK();
+void launch_mm(MmArgs a, const DecState& st, int tiles, hipStream_t s) {
+    const int blocks = cdiv(a.B, 16), per = cdiv(a.chunks, 8);   // chunks of a wave
+    for (a.block0 = 0; a.block0 < blocks; a.block0 += 65535) {
+        const dim3 grid(tiles, std::min(65535, blocks - a.block0));
+        if (per <= 5) launch(dec_mm_kernel<MODE, 5>, grid, dim3(512), 0, s, a, st);
+        else if (per <= 10) launch(dec_mm_kernel<MODE, 10>, grid, dim3(512), 0, s, a, st);
+        else launch(dec_mm_kernel<MODE, 16>, grid, dim3(512), 0, s, a, st);
+        PKX_LAUNCH_CHECK();
+    }
 }
 }  // namespace
 
@@ -399,7 +403,6 @@ void Model::transducer_greedy(const float* enc, int B, int T_max, const int* T_v
     require(n_tok <= pred_.V1, "decode: joint tokens exceed the embedding rows");
     require(H % 4 == 0 && Hj % 4 == 0, "decode: pred_hidden and joint_hidden must be multiples of 4");
     require(H <= 1024 && Hj <= 2048, "decode: pred_hidden above 1024 or joint_hidden above 2048");
-    require(B <= 65535 * 16, "decode: too many items");
     for (int b = 0; b < B; ++b) require(T_valid[b] >= 0 && T_valid[b] <= T_max, "decode: T_valid outside [0, T_max]");
     for (int i = 0; i < n_dur; ++i) require(durations && durations[i] >= 0, "decode: durations must be >= 0");
 

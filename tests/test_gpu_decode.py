@@ -261,3 +261,24 @@ def test_greedy_decode_past_the_kept_workspace(gpu, stream):
         got = gm.transducer_greedy(d_enc, T_valid, durations=durations, cap=400, stream=stream)
         _check_items(got, [tr.greedy(enc[b, :T_valid[b]], durations=durations, max_symbols=10) for b in range(B)])
         d_enc.free()
+
+
+def test_greedy_decode_more_items_than_a_grid_dimension(gpu, stream):
+    """More 16-item blocks than a grid's second dimension holds (1,048,560 items):
+    22 different items over and over, the repeats identical and the first ones
+    the oracle's."""
+    durations = (0, 1, 2, 3, 4)
+    cfg, m = _model(durations, seed=6)
+    gm, tr = gpu.Model.from_tensors(m), oracle.Transducer(m)
+    n, B, cap = 22, 65535 * 16 + 40, 11
+    one = np.random.default_rng(66).standard_normal((n, 1, cfg.d_model)).astype(np.float32)
+    enc = np.concatenate([one] * (B // n) + [one[:B % n]])
+    print(f"[decode] B={B}", flush=True)
+    d_enc = gpu.DeviceArray.from_numpy(enc, stream)
+    (ids, fr, cf, sp), cnt = _raw_greedy(gpu, gm, d_enc, [1] * B, durations, cfg.vocab_size, cap, stream)
+    _check_items([(ids[b, :cnt[b]], fr[b, :cnt[b]], cf[b, :cnt[b]], sp[b, :cnt[b]]) for b in range(n)],
+                 [tr.greedy(one[b], durations=durations, max_symbols=10) for b in range(n)])
+    for a in (ids, fr, cf, sp, cnt[:, None]):
+        rep = a[:B // n * n].reshape(B // n, n, -1)
+        assert (rep == rep[:1]).all() and np.array_equal(a[B // n * n:], a[:B % n])
+    d_enc.free()
