@@ -513,14 +513,14 @@ void MelFront::forward(const float* pcm, int B, int64_t S_stride, const int* n_s
     p.preemph = cfg_.preemph;
     p.mag_power = cfg_.mag_power;
     p.log_guard = cfg_.log_guard;
-    if (cfg_.n_fft != 512 || cfg_.mag_power != 2.0f || fb_nnz_ > MEL_FB_LDS || cfg_.n_mels > MEL_SPAN_LDS) {
+    const int64_t n_groups = (int64_t)cdiv(T_max, 4) * B;
+    if (cfg_.n_fft != 512 || cfg_.mag_power != 2.0f || fb_nnz_ > MEL_FB_LDS || cfg_.n_mels > MEL_SPAN_LDS ||
+        n_groups >= ((int64_t)1 << 31) - (1 << 20)) {   // its group numbers are 32-bit
         launch(mel_spec_kernel, dim3(cdiv(T_max, MEL_FRAMES_PER_BLOCK), B), dim3(256), 0, s, p);
     } else {
         // four workgroups a CU (what their LDS and registers allow), each with its share of the groups
-        const int groups = cdiv(T_max, 4);
-        require((int64_t)groups * B < ((int64_t)1 << 31) - (1 << 20), "mel: too many frames for one call");
-        const int n_groups = groups * B;
-        launch(mel_spec512_kernel, dim3(std::min(n_groups, 4 * device_cu_count())), dim3(256), 0, s, p, groups, n_groups);
+        launch(mel_spec512_kernel, dim3((unsigned)std::min<int64_t>(n_groups, 4 * device_cu_count())), dim3(256), 0, s, p,
+               cdiv(T_max, 4), (int)n_groups);
     }
     PKX_LAUNCH_CHECK();
     const dim3 rows(cfg_.n_mels, B);
