@@ -256,7 +256,9 @@ int pkx_rel_pos_encoding(int T, int D, float* out_dev, void* stream);
  * (host) frames per item.  Outputs (host, [B][cap] each, NULL to skip): token
  * ids, NeMo frame / max_prob confidence / span per token (src/decode_types.hpp);
  * counts (host) [B] tokens per item; the entries past an item's tokens are 0.
- * A decode needing more than cap tokens for an item is an error. */
+ * A decode needing more than cap tokens for an item is an error.  Up to 64 MB of
+ * device memory stay with the model for the next call, until pkx_model_free;
+ * decodes on one model may overlap, from threads and on streams of their own. */
 int pkx_transducer_greedy(pkx_model* m, const float* enc_dev, int B, int T_max, const int* T_valid,
                           const int32_t* durations, int n_durations, int blank_id, int max_symbols, int cap,
                           int32_t* ids, int32_t* frames, float* conf, int32_t* span, int* counts, void* stream);
